@@ -1,34 +1,33 @@
-// Pointwise (1x1) convolutions over flat planes of N pixels, as split f16
-// products (split.h): the SpectralTransform's conv1 and FourierUnit conv
-// (lama_conv1x1*), and conv2 with the l2g addend, BN_g, ReLU and the residual
-// fused (lama_conv1x1_res*).
+// Pointwise (1x1) convolutions over flat planes of N pixels, on three bf16 parts
+// (split.h): the SpectralTransform's conv1 and FourierUnit conv (lama_conv1x1*),
+// and conv2 with the l2g addend, BN_g, ReLU and the residual fused
+// (lama_conv1x1_res*).
 //
 // A workgroup computes MB output channels x NPX pixels.  Its input strip is
 // taken in fills of KC channels: every thread loads PER runs of 8 channels of
 // one pixel (a wave's loads are whole 128- or 256-byte lines of a plane,
-// whatever its alignment or stride), the workgroup agrees on the strip's
-// scale, and each run becomes one 16-byte store of its 8 his and one of its 8
-// los into LDS, [part][8-channel group][pixel][8]: the lanes of a wave write,
-// and of an MFMA operand read, consecutive 16-byte words.  The next fill's
-// loads are in flight meanwhile.  Weights are MFMA operands of one wave each,
-// packed in operand order ([32 channels][8-channel group][part][32][8]) and
-// loaded straight into registers, RING 16-channel steps ahead.  Two waves share
-// 32 channels and take every second step each (K halves); their sums meet in
-// LDS, and each finishes half the rows.
+// whatever its alignment or stride), and each run becomes one 16-byte store of
+// each of its three parts into LDS, [part][8-channel group][pixel][8]: the lanes
+// of a wave write, and of an MFMA operand read, consecutive 16-byte words.  The
+// next fill's loads are in flight meanwhile.  Weights are MFMA operands of one
+// wave each, packed in operand order ([32 channels][8-channel group][part][32][8])
+// and loaded straight into registers, RING 16-channel steps ahead.  Two waves
+// share 32 channels and take every second step each (K halves); their sums meet
+// in LDS, and each finishes half the rows.
 //
-// lama_conv1x1_kh, lama_conv1x1_res_kh: 96 channels x 32 pixels, K = 384 (192)
-// in one fill.  For the planes whose 64 x 64 tiles would give at most two
-// workgroups per CU (Engine::tile_variant): what bounds them is the latency of
-// one strip, load to store, and the bytes a CU takes through its L1 meanwhile;
-// conv1 at 64 x 64 is 256 workgroups, one a CU, of 196 KB each (64 x 32 tiles:
-// 1.5 a CU of 147 KB, 8.0 us against 6.4).  At most 128 registers, so that two
-// six-wave workgroups fit a CU.  64 x 64 plane, conv1 / FU / conv2 alone:
-// 11.6 / 11.8 / 10.0 us with f32 MFMAs, 6.4 / 8.0 / 7.3 now.
+// lama_conv1x1_kh, lama_conv1x1_res_kh: 96 channels x 32 pixels in fills of 192,
+// for the planes whose 64 x 64 tiles would give at most two workgroups per CU
+// (Engine::tile_variant): what bounds them is the latency of one strip, load to
+// store, and the bytes a CU takes through its L1 meanwhile; conv1 at 64 x 64 is
+// 256 workgroups, one a CU.  At most 128 registers, so that two six-wave
+// workgroups fit a CU and one beside the FFC GEMM's (168: 15.0 us against 11.5 in
+// a 512 x 512 pass; K = 384 in one fill, 73 KB of LDS: 14.4).  Alone, f32 MFMAs /
+// here: conv1 at 64 x 64 14.0 / 11.3 us, the FU conv 11.2 / 10.2 and 14.4 / 13.9
+// at 192 and 384 channels.
 // lama_conv1x1, lama_conv1x1_res: 64 channels x 64 pixels in fills of 96, the
 // larger planes, where the weights feed twice the pixels and three workgroups a
-// CU cover each other's loads.  256 x 256 plane, alone: conv1 107 -> 55 us,
-// conv2 130 -> 105 (192-channel tiles of six waves: 107 and 147; one of them a
-// CU).
+// CU cover each other's loads.  256 x 256 plane, alone: conv1 106.7 / 82.3 us
+// (in a 1024 x 1024 pass 47 us; 96-channel tiles of six waves 52).
 #include <hip/hip_runtime.h>
 
 #include "common.h"
@@ -51,7 +50,7 @@ struct PwCfg {
     static constexpr int RING = WS % 4 == 0 ? 4 : 3;        // weight steps in registers
     static constexpr int PER = KG * NPX / NT, GPR = NT / NPX;  // runs per thread; groups per round of runs
     static constexpr int GPW = 64 / NPX;                    // groups per wave of a round
-    static constexpr int XL = 2 * KG * NPX;                 // LDS h8s: his, then los
+    static constexpr int XP = KG * NPX, XL = 3 * XP;        // LDS b8s of one part, of the three
     static_assert(PER * NT == KG * NPX && (NPX == 32 || NPX == 64), "whole runs");
     static_assert(WS % RING == 0, "the ring holds a whole number of laps per fill");
     static_assert(!KH || MW * NCB * 16 * 64 * 4 <= XL * 16, "the halves' exchange fits the strip's LDS");
@@ -65,7 +64,7 @@ struct PwCfg {
 // partial at out + ks * out_kstride (the host clears bias, BN, ReLU, addends
 // and residual; the consumer sums the partials and applies them).
 template <class C, bool RES>
-__device__ __forceinline__ void pw_tile(const ConvProblem &P_mem, int b, h8 *xs, float *slot, float *epl)
+__device__ __forceinline__ void pw_tile(const ConvProblem &P_mem, int b, b8 *xs, float *epl)
 {
     const ConvProblem P = P_mem;  // one batch of scalar loads, held across the barriers
     int ks = 0;
@@ -104,7 +103,7 @@ __device__ __forceinline__ void pw_tile(const ConvProblem &P_mem, int b, h8 *xs,
     if (P.ksplit > 1) {
         const int c0 = ks * P.kchunks * 16;
         src += (long)c0 * cs;
-        wt += (long)c0 / 8 * 256;
+        wt += (long)c0 / 8 * 384;
         n16 = P.kchunks;
         nc = min(nc - c0, n16 * 16);
     }
@@ -116,120 +115,72 @@ __device__ __forceinline__ void pw_tile(const ConvProblem &P_mem, int b, h8 *xs,
     const unsigned xoff = 4u * ((unsigned)px + (C::NPX == 32 ? 8u * (unsigned)g * (unsigned)cs : 0u));
     const int wgrp = C::NPX == 32 ? 2 * wave : wave;
     float r[C::PER][8];
-    // a fill whose channels are whole runs of every wave goes through
-    // registers (zeros past them), any other through the loops below
-    auto whole = [&](int f) { return min(C::KC, nc - f * C::KC) % (8 * C::GPW) == 0; };
     auto load = [&](int f) {
         const int nk = nc - f * C::KC;
+        if (min(C::KC, nk) % (8 * C::GPW) == 0) {  // whole runs of every wave; zeros past them
 #pragma unroll
-        for (int it = 0; it < C::PER; ++it)
-            if (8 * (it * C::GPR + wgrp) < nk) {
-                const LAMA_GLOBAL float *p = src + (long)(f * C::KC + 8 * (it * C::GPR + wgrp)) * cs;
+            for (int it = 0; it < C::PER; ++it)
+                if (8 * (it * C::GPR + wgrp) < nk) {
+                    const LAMA_GLOBAL float *p = src + (long)(f * C::KC + 8 * (it * C::GPR + wgrp)) * cs;
 #pragma unroll
-                for (int e = 0; e < 8; ++e, p += cs) r[it][e] = *at_byte<float>(p, xoff);
-            } else {
+                    for (int e = 0; e < 8; ++e, p += cs) r[it][e] = *at_byte<float>(p, xoff);
+                } else {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) r[it][e] = 0.f;
-            }
+                    for (int e = 0; e < 8; ++e) r[it][e] = 0.f;
+                }
+        } else {  // a ragged channel count, value by value
+#pragma unroll
+            for (int it = 0; it < C::PER; ++it)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int c = 8 * (it * C::GPR + wgrp + (C::NPX == 32 ? g : 0)) + e;
+                    const float v = src[(long)(f * C::KC + min(c, nk - 1)) * cs + px];
+                    r[it][e] = c < nk ? v : 0.f;
+                }
+        }
     };
-    if (whole(0)) load(0);
+    load(0);
     // weights: lane (g, j) takes row j and group 2 k16 + g
-    h8 wh[C::RING], wl[C::RING];
-    const unsigned woff = (unsigned)(g * 1024 + j * 16);
+    b8 w0[C::RING], w1[C::RING], w2[C::RING];
+    const unsigned woff = (unsigned)(g * 1536 + j * 16);
     auto load_w = [&](int sl, int f, int s) {
         const int k16 = min(f * C::KS + (C::KH ? 2 * s + kh : s), n16 - 1);
-        const LAMA_GLOBAL float *p = wt + (long)k16 * 512;
-        wh[sl] = *at_byte<h8>(p, woff);
-        wl[sl] = *at_byte<h8>(p, woff + 512u);
+        const LAMA_GLOBAL float *p = wt + (long)k16 * 768;
+        w0[sl] = *at_byte<b8>(p, woff);
+        w1[sl] = *at_byte<b8>(p, woff + 512u);
+        w2[sl] = *at_byte<b8>(p, woff + 1024u);
     };
 #pragma unroll
     for (int s = 0; s < C::RING; ++s) load_w(s, 0, s);
     // per-channel epilogue operands: loaded here, parked in LDS with the first fill
-    float ep[4];
+    float ep[3];
     {
         const int c = min(m0 + min(tid, C::MB - 1), P.M - 1);
         ep[0] = P.bias ? gp(P.bias)[c] : 0.f;
         ep[1] = P.scale ? gp(P.scale)[c] : 1.f;
         ep[2] = P.scale ? gp(P.shift)[c] : 0.f;
-        ep[3] = gp(sg.wsc)[c];
     }
-    f32x16 acc[C::NCB];
+    f32x16 acc[C::NCB], low[C::NCB];
 #pragma unroll
     for (int h = 0; h < C::NCB; ++h)
 #pragma unroll
-        for (int q = 0; q < 16; ++q) acc[h][q] = 0.f;
-    int k = SPLIT_K_START;
-    for (int f = 0; f < nf; ++f) {
-        float m = 0.f;
+        for (int q = 0; q < 16; ++q) acc[h][q] = low[h][q] = 0.f;
+    auto stage = [&](auto any) {
+        float check = 0.f;
 #pragma unroll
-        for (int it = 0; it < C::PER; ++it)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(r[it][e]));
-        m = wave_max(whole(f) ? m : __builtin_inff());
-        auto agree = [&](float v) {  // the workgroup's largest
-            if (lane == 0) slot[wave] = v;
-            __syncthreads();  // and every wave is done with the last fill's strip
-            float mm = 0.f;
-#pragma unroll
-            for (int w = 0; w < C::WAVES; ++w) mm = fmaxf(mm, slot[w]);
-            return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(mm)));
-        };
-        float mm = agree(m);
-        auto rescale = [&]() {
-            const int kn = split_exp(k, mm, 0);
-            if (kn != k) {
-                if (f > 0) {
-                    const float d = pow2f(max(kn - k, -126));
-#pragma unroll
-                    for (int h = 0; h < C::NCB; ++h)
-#pragma unroll
-                        for (int e = 0; e < 16; ++e) acc[h][e] *= d;
-                }
-                k = kn;
-            }
-        };
-        if (mm < __builtin_inff()) {
-            rescale();
-            const float s = pow2f(k);
-#pragma unroll
-            for (int it = 0; it < C::PER; ++it) {
-                h8 hi, lo;
-                split_n<false>(r[it], s, hi, lo);
-                xs[tid + it * C::NT] = hi;  // [group][pixel]
-                xs[tid + it * C::NT + C::KG * C::NPX] = lo;
-            }
-        } else {
-            // a ragged channel count, infinities or NaNs: value by value, the
-            // scale that of the finite ones
-            const int c0 = f * C::KC, nv = min(C::KC, nc - c0) * C::NPX;
-            auto value = [&](int i) { return src[(long)(c0 + i / C::NPX) * cs + min(ox0 + i % C::NPX, N - 1)]; };
-            m = 0.f;
-#pragma nounroll
-            for (int i = tid; i < nv; i += C::NT) {
-                const float a = fabsf(value(i));
-                m = fmaxf(m, a < __builtin_inff() ? a : 0.f);
-            }
-            m = wave_max(m);
-            __syncthreads();
-            mm = agree(m);
-            rescale();
-            const float s = pow2f(k);
-            _Float16 *xe = reinterpret_cast<_Float16 *>(xs);
-#pragma nounroll
-            for (int i = tid; i < C::KC * C::NPX; i += C::NT) {
-                const int c = i / C::NPX;
-                const float v[2] = {i < nv ? value(i) : 0.f, 0.f};
-                h2 hi, lo;
-                split_n<true>(v, s, hi, lo);
-                const int at = ((c >> 3) * C::NPX + i % C::NPX) * 8 + (c & 7);
-                xe[at] = hi[0];
-                xe[at + C::KG * C::NPX * 8] = lo[0];
-            }
+        for (int it = 0; it < C::PER; ++it) {
+            b8 *to = xs + tid + it * C::NT;  // [part][group][pixel]
+            check += split3<decltype(any)::value>(r[it], to[0], to[C::XP], to[2 * C::XP]);
         }
+        return check;
+    };
+    for (int f = 0; f < nf; ++f) {
+        if (f > 0) __syncthreads();  // every wave is done with the last fill's strip
+        if (split3_again(stage(std::false_type{}))) stage(std::true_type{});
         if (f == 0 && tid < C::MB)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) epl[i * C::MB + tid] = ep[i];
-        if (f + 1 < nf && whole(f + 1)) load(f + 1);
+            for (int i = 0; i < 3; ++i) epl[i * C::MB + tid] = ep[i];
+        if (f + 1 < nf) load(f + 1);
         __syncthreads();
         // laps of the ring; the steps of a lap past the last channel multiply zeros
 #pragma unroll
@@ -238,10 +189,11 @@ __device__ __forceinline__ void pw_tile(const ConvProblem &P_mem, int b, h8 *xs,
 #pragma unroll
             for (int i = 0; i < C::RING; ++i) {
                 const int s = lap + i;
-                const h8 *x = xs + (2 * (C::KH ? 2 * s + kh : s) + g) * C::NPX + j;
+                const b8 *x = xs + (2 * (C::KH ? 2 * s + kh : s) + g) * C::NPX + j;
 #pragma unroll
                 for (int h = 0; h < C::NCB; ++h)
-                    acc[h] = mfma_split(wh[i], wl[i], x[32 * h], x[32 * h + C::KG * C::NPX], acc[h]);
+                    mfma_split3(w0[i], w1[i], w2[i], x[32 * h], x[32 * h + C::XP], x[32 * h + 2 * C::XP], acc[h],
+                                low[h]);
                 // this step's registers: the step RING on, here or in the next fill
                 if (s + C::RING < C::WS)
                     load_w(i, f, s + C::RING);
@@ -250,9 +202,10 @@ __device__ __forceinline__ void pw_tile(const ConvProblem &P_mem, int b, h8 *xs,
             }
         }
     }
-    const float u = pow2f(-k);  // |k| <= 100 once a fill has been taken
+#pragma unroll
+    for (int h = 0; h < C::NCB; ++h) acc[h] += low[h];
     // K halves: each of the two waves finishes eight of the 16 register rows,
-    // handing the other eight (in the common scale) over
+    // handing the other eight over
     if constexpr (C::KH) {
         float *ex = reinterpret_cast<float *>(xs) + wm * C::NCB * 16 * 64 + lane;
         __syncthreads();
@@ -303,7 +256,7 @@ __device__ __forceinline__ void pw_tile(const ConvProblem &P_mem, int b, h8 *xs,
             for (int q = 0; q < NQ; ++q) {
                 const int cl = row0 - m0 + 4 * g + 8 * (q >> 2) + (q & 3);
                 // absent operands are neutral (0, 1, 0): no branch a value
-                float v = acc[h][q] * epl[3 * C::MB + cl] * u + epl[cl];
+                float v = acc[h][q] + epl[cl];
                 if constexpr (RES) v += add[q];
                 v = v * epl[C::MB + cl] + epl[2 * C::MB + cl];
                 v = P.relu ? fmaxf(v, 0.f) : v;
@@ -328,15 +281,15 @@ __device__ __forceinline__ void pw_tile(const ConvProblem &P_mem, int b, h8 *xs,
         LAMA_CONV_STARTS;                                                                               \
         LAMA_STAMP_BEGIN;                                                                               \
         using C = PwCfg<NPX, MW, KH, KC>;                                                               \
-        __shared__ h8 xs[C::XL];                                                                        \
-        __shared__ float slot[C::WAVES], epl[4 * C::MB];                                                \
+        __shared__ b8 xs[C::XL];                                                                        \
+        __shared__ float epl[3 * C::MB];                                                                \
         int b = blockIdx.x;                                                                             \
         const int pi = find_problem(ps, b);                                                             \
-        pw_tile<C, RES>(probs[pi], b, xs, slot, epl);                                                   \
+        pw_tile<C, RES>(probs[pi], b, xs, epl);                                                         \
         LAMA_STAMP_END;                                                                                 \
     }
 LAMA_PW_KERNEL(lama_conv1x1, 64, LAMA_PW_MB / 32, true, LAMA_PW_KC, false)
-LAMA_PW_KERNEL(lama_conv1x1_kh, 32, LAMA_PW_KH_MB / 32, true, 384, false)
+LAMA_PW_KERNEL(lama_conv1x1_kh, 32, LAMA_PW_KH_MB / 32, true, 192, false)
 LAMA_PW_KERNEL(lama_conv1x1_res, 64, LAMA_PW_MB / 32, true, LAMA_PW_KC, true)
 LAMA_PW_KERNEL(lama_conv1x1_res_kh, 32, LAMA_PW_KH_MB / 32, true, 192, true)
 #undef LAMA_PW_KERNEL

@@ -425,9 +425,38 @@ Packed pack_tail(Arena &A, int C, const float *w)
     return p;
 }
 
-// Pointwise weights [M][C] for the split-product kernels: [32 rows][group of 8
-// channels][hi, lo][32][8] halves, rows past M and channels past C zero, the
-// groups rounded up to whole 16-channel steps; the row scales beside them.
+// v as three bf16 parts, out[0], out[stride] and out[2 stride] (split.h): each
+// the nearest to what the ones before leave, the first towards zero where the
+// nearest would be infinite; infinities and NaNs whole in the third.
+void split_bf16(float v, uint16_t *out, size_t stride)
+{
+    auto bits = [](float x) {
+        uint32_t u;
+        std::memcpy(&u, &x, 4);
+        return u;
+    };
+    auto value = [](uint32_t u) {
+        float x;
+        std::memcpy(&x, &u, 4);
+        return x;
+    };
+    uint32_t u = bits(v);
+    if ((u & 0x7fffffff) >= 0x7f800000) {
+        out[0] = out[stride] = 0;
+        out[2 * stride] = (uint16_t)(u >> 16 | ((u & 0x7fffff) ? 0x40 : 0));
+        return;
+    }
+    for (int i = 0; i < 3; ++i, out += stride) {
+        uint32_t r = (u + 0x7fff + (u >> 16 & 1)) & 0xffff0000;  // to nearest, ties to even
+        if ((r & 0x7fffffff) == 0x7f800000) r = u & 0xffff0000;
+        *out = (uint16_t)(r >> 16);
+        u = bits(value(u) - value(r));
+    }
+}
+
+// Pointwise weights [M][C] for the kernels in three bf16 parts: [32 rows][group
+// of 8 channels][part][32][8], rows past M and channels past C zero, the groups
+// rounded up to whole 16-channel steps.
 template <class Get>
 Packed pack_pw(Arena &A, int M, int C, const Get &get)
 {
@@ -437,21 +466,12 @@ Packed pack_pw(Arena &A, int M, int C, const Get &get)
     p.T = 1;
     p.KC = 16;
     p.nchunk = (C + 15) / 16;
-    p.wrow = p.nchunk * 16;
+    p.wrow = p.nchunk * 24;
     p.off = A.add((size_t)((M + 31) / 32) * 32 * p.wrow);
-    p.ws = A.add(M);
     uint16_t *d = reinterpret_cast<uint16_t *>(A.at(p.off));
     for (int co = 0; co < M; ++co) {
-        float most = 0;
-        for (int ci = 0; ci < C; ++ci)
-            if (std::isfinite(get(co, ci))) most = std::max(most, std::fabs(get(co, ci)));
-        const int e = split_row_exp(most);
-        A.at(p.ws)[co] = std::ldexp(1.f, -e);
         uint16_t *blk = d + (size_t)(co / 32) * 64 * p.wrow + (co % 32) * 8;
-        for (int ci = 0; ci < C; ++ci) {
-            uint16_t *g = blk + (size_t)(ci / 8) * 512 + ci % 8;
-            split_f16(get(co, ci), e, g[0], g[256]);
-        }
+        for (int ci = 0; ci < C; ++ci) split_bf16(get(co, ci), blk + (size_t)(ci / 8) * 768 + ci % 8, 256);
     }
     return p;
 }
