@@ -1,28 +1,26 @@
 // The 7x7 head (model.1, at the end), the stride-2 3x3 convolutions (model.2/3/4)
-// and the transposed ones (model.24/27/30) as implicit GEMMs on split f16
-// products (split.h).
+// and the transposed ones (model.24/27/30) as implicit GEMMs on three bf16 parts
+// (split.h).
 //
 // A workgroup computes 64 output channels x 128 GEMM pixels (TR rows of TC; for
 // the transposed convolutions, 128 input positions of one row phase py, both
 // column phases: output rows 2m+py).  Wave (wm, wn) owns 32 channels and 64
 // pixels, two 32 x 32 accumulators a phase, so that a weight operand feeds 64
-// pixels: with 32 the four waves would ask their CU's L1 for 85 bytes a cycle
-// at full MFMA rate, which gives 64.  K is walked in chunks of 16 channels x T
-// taps.  The chunk's input patch, loaded into registers during the chunk
-// before, is scaled, split and stored as [part][8-channel group][pixel][8]
-// halves, so that an MFMA operand of a tap is one 16-byte read a lane over
-// consecutive pixels; a stride-2 patch row keeps its even and its odd columns
-// in two runs, so that output pixels' inputs are consecutive there too.  The
-// im2col matrix is never formed; reflect padding is an index map.  Weights are
-// MFMA operands in operand order ([32 rows][8-channel group][tap][part][32][8])
-// and go straight into registers, a chunk ahead.
+// pixels.  K is walked in chunks of 16 channels x T taps.  The chunk's input
+// patch, loaded into registers during the chunk before, is split and stored as
+// [part][8-channel group][pixel][8], so that an MFMA operand of a tap is one
+// 16-byte read a lane over consecutive pixels; a stride-2 patch row keeps its
+// even and its odd columns in two runs, so that output pixels' inputs are
+// consecutive there too.  The im2col matrix is never formed; reflect padding is
+// an index map.  Weights are MFMA operands in operand order ([32 rows][8-channel
+// group][tap][part][32][8]) and go straight into registers, three taps ahead (a
+// whole chunk ahead, at 234 registers: 981 us against 895 for the stride-2 ones
+// at 2048x2048).
 //
-// What bounds it: at 2048x2048 memory, not yet at its rate (model.2 reads and
-// writes 1.6 GB, 333 us at a copy's 4.8 TB/s; the loads of one chunk in flight
-// do not cover the latency at two workgroups a CU); at 512x512 too few
-// workgroups (128 to 512) for that.  One launch (median of the three), f32
-// MFMAs -> split, us: stride 2 at 512x512 87 -> 40, at 2048x2048 1370 -> 577;
-// transposed 88 -> 43 and 1230 -> 567.
+// What bounds it: the six MFMAs a product (model.2 at 2048x2048: 370 us at the
+// bf16 peak) and the latency of staging between them, at two workgroups a CU.
+// One launch (mean of the three), f32 MFMAs / here, us: stride 2 at 512x512 96 /
+// 61, at 2048x2048 1370 / 910; transposed 93 / 65 and 1230 / 806.
 #include <hip/hip_runtime.h>
 
 #include "common.h"
@@ -46,7 +44,7 @@ struct EdgeCfg {
     static constexpr int PR = DOWN ? 2 * TR + 1 : TR + PY, PC = DOWN ? 2 * TC + 1 : TC + 1;
     static constexpr int HPC = (PC + 1) / 2, PCP = DOWN ? 2 * HPC : PC;  // columns a row holds in LDS
     static constexpr int NP = PR * PC, HT = LAMA_NT / 2, PER = (NP + HT - 1) / HT;
-    static constexpr int GS = PR * PCP, PS = 2 * GS, LDS = 2 * PS;  // group and part strides, in h8
+    static constexpr int GS = PR * PCP, PS = 2 * GS, LDS = 3 * PS;  // group and part strides, in b8
     static __device__ __forceinline__ constexpr int col(int c) { return DOWN ? (c & 1) * HPC + (c >> 1) : c; }
     static __device__ __forceinline__ constexpr int dy(int t) { return DOWN ? t / 3 : PY && (t == 1 || t >= 4) ? 1 : 0; }
     static __device__ __forceinline__ constexpr int dx(int t)
@@ -58,7 +56,7 @@ struct EdgeCfg {
 };
 
 template <class C>
-__device__ __forceinline__ void edge_tile(const ConvProblem &P_mem, int b, h8 *xs, float *slot, float *epl)
+__device__ __forceinline__ void edge_tile(const ConvProblem &P_mem, int b, b8 *xs, float *epl)
 {
     const ConvProblem P = P_mem;  // one batch of scalar loads, held across the barriers
     const int mb = b % P.mblocks, t_ = b / P.mblocks;
@@ -106,35 +104,45 @@ __device__ __forceinline__ void edge_tile(const ConvProblem &P_mem, int b, h8 *x
     };
     load(0);
     // lane (g, j): row j of the wave's 32, group 2 ck + g (past the last: the last, against zeros)
-    h8 wh[C::T], wl[C::T];
+    constexpr int RING = 3;
+    b8 w0[RING], w1[RING], w2[RING];
     auto load_w = [&](int t, int ck) {
-        const unsigned o = (unsigned)(min(2 * ck + g, ng - 1) * (C::T * 1024) + j * 16);
-        const LAMA_GLOBAL float *p = wt + t * 256;
-        wh[t] = *at_byte<h8>(p, o);
-        wl[t] = *at_byte<h8>(p, o + 512u);
+        const unsigned o = (unsigned)(min(2 * ck + g, ng - 1) * (C::T * 1536) + j * 16);
+        const LAMA_GLOBAL float *p = wt + t * 384;
+        w0[t % RING] = *at_byte<b8>(p, o);
+        w1[t % RING] = *at_byte<b8>(p, o + 512u);
+        w2[t % RING] = *at_byte<b8>(p, o + 1024u);
     };
 #pragma unroll
-    for (int t = 0; t < C::T; ++t) load_w(t, 0);
+    for (int t = 0; t < RING; ++t) load_w(t, 0);
     const int ec = min(m0 + (tid & 63), P.M - 1);
     const float ep = tid < 64    ? (P.bias ? gp(P.bias)[ec] : 0.f)
                      : tid < 128 ? (P.scale ? gp(P.scale)[ec] : 1.f)
-                     : tid < 192 ? (P.scale ? gp(P.shift)[ec] : 0.f)
-                                 : gp(sg.wsc)[ec];
-    f32x16 acc[C::NPH][2];
+                                 : (P.scale ? gp(P.shift)[ec] : 0.f);
+    f32x16 acc[C::NPH][2], low[C::NPH][2];
 #pragma unroll
     for (int p = 0; p < C::NPH; ++p)
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[p][h][r] = 0.f;
+            for (int r = 0; r < 16; ++r) acc[p][h][r] = low[p][h][r] = 0.f;
     // the wave's two runs of 32 pixels
-    const h8 *rd[2];
+    const b8 *rd[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const int p = wn * 64 + h * 32 + j;
         rd[h] = xs + g * C::GS + (p / C::TC) * C::S * C::PCP + p % C::TC;
     }
-    int k = SPLIT_K_START;
+    auto stage = [&](auto any) {
+        float check = 0.f;
+#pragma unroll
+        for (int it = 0; it < C::PER; ++it) {
+            if (it == C::PER - 1 && C::NP % C::HT && it0 + it * C::HT >= C::NP) break;
+            b8 *to = xs + pl[it];
+            check += split3<decltype(any)::value>(d[it], to[0], to[C::PS], to[2 * C::PS]);
+        }
+        return check;
+    };
     for (int ck = 0; ck < n; ++ck) {
         if (!C::DOWN || (ck + 1) * C::KC > nc) {
 #pragma unroll
@@ -144,65 +152,19 @@ __device__ __forceinline__ void edge_tile(const ConvProblem &P_mem, int b, h8 *x
                     if (!(in >> it & 1u) || ck * C::KC + 8 * ig + e >= nc) d[it][e] = 0.f;
             }
         }
-        auto agree = [&](bool finite) {  // the workgroup's largest magnitude
-            float m = 0.f;
-#pragma unroll
-            for (int it = 0; it < C::PER; ++it)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float a = fabsf(d[it][e]);
-                    m = fmaxf(m, finite && !(a < __builtin_inff()) ? 0.f : a);
-                }
-            m = wave_max(m);
-            if (lane == 0) slot[wave] = m;
-            __syncthreads();  // and every wave is done with the last chunk's operands
-            m = fmaxf(fmaxf(slot[0], slot[1]), fmaxf(slot[2], slot[3]));
-            return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(m)));
-        };
-        float m = agree(false);
-        const bool inf = !(m < __builtin_inff());
-        if (inf) {  // the scale is that of the finite values
-            __syncthreads();
-            m = agree(true);
-        }
-        const int kn = split_exp(k, m, 0);
-        if (kn != k) {
-            if (ck > 0) {
-                const float f = pow2f(max(kn - k, -126));
-#pragma unroll
-                for (int p = 0; p < C::NPH; ++p)
-#pragma unroll
-                    for (int h = 0; h < 2; ++h)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) acc[p][h][r] *= f;
-            }
-            k = kn;
-        }
-        const float s = pow2f(k);
-        auto store = [&](auto inf_) {
-#pragma unroll
-            for (int it = 0; it < C::PER; ++it) {
-                if (it == C::PER - 1 && C::NP % C::HT && it0 + it * C::HT >= C::NP) break;
-                h8 hi, lo;
-                split_n<decltype(inf_)::value>(d[it], s, hi, lo);
-                xs[pl[it]] = hi;
-                xs[pl[it] + C::PS] = lo;
-            }
-        };
-        if (inf)
-            store(std::true_type{});
-        else
-            store(std::false_type{});
+        if (ck > 0) __syncthreads();  // every wave is done with the last chunk's operands
+        if (split3_again(stage(std::false_type{}))) stage(std::true_type{});
         load(min(ck + 1, n - 1));  // unconditional: the waits then count exactly
         __syncthreads();
         // each tap's operand reads are issued before the tap before it
-        h8 xh[2][2], xl[2][2];
+        b8 x0_[2][2], x1_[2][2], x2_[2][2];
         auto read = [&](int t) {
             const int o = C::dy(t) * C::PCP + C::col(C::dx(t));
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                xh[t & 1][h] = rd[h][o];
-                xl[t & 1][h] = rd[h][o + C::PS];
+                x0_[t & 1][h] = rd[h][o];
+                x1_[t & 1][h] = rd[h][o + C::PS];
+                x2_[t & 1][h] = rd[h][o + 2 * C::PS];
             }
         };
         read(0);
@@ -211,16 +173,23 @@ __device__ __forceinline__ void edge_tile(const ConvProblem &P_mem, int b, h8 *x
             if (t + 1 < C::T) read(t + 1);
 #pragma unroll
             for (int h = 0; h < 2; ++h)
-                acc[C::px(t)][h] = mfma_split(wh[t], wl[t], xh[t & 1][h], xl[t & 1][h], acc[C::px(t)][h]);
-            load_w(t, min(ck + 1, n - 1));
+                mfma_split3(w0[t % RING], w1[t % RING], w2[t % RING], x0_[t & 1][h], x1_[t & 1][h], x2_[t & 1][h], acc[C::px(t)][h],
+                            low[C::px(t)][h]);
+            if (t + RING < C::T)
+                load_w(t + RING, ck);
+            else
+                load_w(t + RING - C::T, min(ck + 1, n - 1));
             // keep the load here: the scheduler would otherwise sink it below
             // the chunk's last MFMA
             __builtin_amdgcn_sched_barrier(0);
         }
     }
-    epl[tid] = ep;
+#pragma unroll
+    for (int p = 0; p < C::NPH; ++p)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) acc[p][h] += low[p][h];
+    if (tid < 192) epl[tid] = ep;
     __syncthreads();
-    const float u = pow2f(-k);  // |k| <= 100 once a chunk has been taken
     const int row0 = wm * 32 + 4 * g;  // register r: channel m0 + row0 + 8 (r / 4) + r % 4
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -235,7 +204,7 @@ __device__ __forceinline__ void edge_tile(const ConvProblem &P_mem, int b, h8 *x
             float v[C::NPH];
 #pragma unroll
             for (int q = 0; q < C::NPH; ++q) {
-                v[q] = acc[q][h][r] * epl[192 + cl] * u + epl[cl];
+                v[q] = acc[q][h][r] + epl[cl];
                 v[q] = v[q] * epl[64 + cl] + epl[128 + cl];
                 v[q] = P.relu ? fmaxf(v[q], 0.f) : v[q];
             }
@@ -251,11 +220,11 @@ template <int TR, int TC>
 __device__ __forceinline__ void down_body(const ConvProblem *__restrict__ probs, const ProbStarts &ps)
 {
     using C = EdgeCfg<0, TR, TC>;
-    __shared__ h8 xs[C::LDS];
-    __shared__ float slot[4], epl[256];
+    __shared__ b8 xs[C::LDS];
+    __shared__ float epl[192];
     int b = blockIdx.x;
     const int pi = find_problem(ps, b);
-    edge_tile<C>(probs[pi], conv_xcd_order(b, probs[pi].nblocks), xs, slot, epl);
+    edge_tile<C>(probs[pi], conv_xcd_order(b, probs[pi].nblocks), xs, epl);
 }
 
 template <int TR, int TC>
@@ -263,16 +232,16 @@ __device__ __forceinline__ void up_body(const ConvProblem *__restrict__ probs, c
 {
     using C0 = EdgeCfg<1, TR, TC>;
     using C1 = EdgeCfg<2, TR, TC>;
-    __shared__ h8 xs[C1::LDS];
-    __shared__ float slot[4], epl[256];
+    __shared__ b8 xs[C1::LDS];
+    __shared__ float epl[192];
     static_assert(C0::LDS <= C1::LDS, "one LDS layout");
     int b = blockIdx.x;
     const int pi = find_problem(ps, b);
     b = conv_xcd_order(b, probs[pi].nblocks);
     if (pi == 0)
-        edge_tile<C0>(probs[0], b, xs, slot, epl);
+        edge_tile<C0>(probs[0], b, xs, epl);
     else
-        edge_tile<C1>(probs[1], b, xs, slot, epl);
+        edge_tile<C1>(probs[1], b, xs, epl);
 }
 
 }  // namespace

@@ -323,10 +323,38 @@ void split_f16(float v, int e, uint16_t &hi, uint16_t &lo)
     lo = f16_bits(x - f16_value(hi));
 }
 
-// Weights of a direct convolution with T taps for the split-product kernels
-// (lama_conv3x3s2, lama_convt_rows): [32 rows][group of 8 channels][tap][hi, lo]
-// [32][8] halves, rows past M and channels past C zero; the row scales beside
-// them.
+// v as three bf16 parts, out[0], out[stride] and out[2 stride] (split.h): each
+// the nearest to what the ones before leave, the first towards zero where the
+// nearest would be infinite; infinities and NaNs whole in the third.
+void split_bf16(float v, uint16_t *out, size_t stride)
+{
+    auto bits = [](float x) {
+        uint32_t u;
+        std::memcpy(&u, &x, 4);
+        return u;
+    };
+    auto value = [](uint32_t u) {
+        float x;
+        std::memcpy(&x, &u, 4);
+        return x;
+    };
+    uint32_t u = bits(v);
+    if ((u & 0x7fffffff) >= 0x7f800000) {
+        out[0] = out[stride] = 0;
+        out[2 * stride] = (uint16_t)(u >> 16 | ((u & 0x7fffff) ? 0x40 : 0));
+        return;
+    }
+    for (int i = 0; i < 3; ++i, out += stride) {
+        uint32_t r = (u + 0x7fff + (u >> 16 & 1)) & 0xffff0000;  // to nearest, ties to even
+        if ((r & 0x7fffffff) == 0x7f800000) r = u & 0xffff0000;
+        *out = (uint16_t)(r >> 16);
+        u = bits(value(u) - value(r));
+    }
+}
+
+// Weights of a direct convolution with T taps for the kernels in three bf16
+// parts (lama_conv3x3s2, lama_convt_rows): [32 rows][group of 8 channels][tap]
+// [part][32][8], rows past M and channels past C zero.
 template <class Get>
 Packed pack_taps(Arena &A, int M, int C, int T, const Get &get)
 {
@@ -336,25 +364,15 @@ Packed pack_taps(Arena &A, int M, int C, int T, const Get &get)
     p.T = T;
     p.KC = 8;
     p.nchunk = (C + 7) / 8;
-    p.wrow = p.nchunk * 8 * T;
+    p.wrow = p.nchunk * 12 * T;
     p.off = A.add((size_t)((M + 31) / 32) * 32 * p.wrow);
-    p.ws = A.add(M);
     uint16_t *d = reinterpret_cast<uint16_t *>(A.at(p.off));
-    float *ws = A.at(p.ws);
     parallel_rows(M, [&](int r0, int r1) {
         for (int co = r0; co < r1; ++co) {
-            float most = 0;
-            for (int ci = 0; ci < C; ++ci)
-                for (int t = 0; t < T; ++t)
-                    if (std::isfinite(get(co, ci, t))) most = std::max(most, std::fabs(get(co, ci, t)));
-            const int e = split_row_exp(most);
-            ws[co] = std::ldexp(1.f, -e);
             uint16_t *blk = d + (size_t)(co / 32) * 64 * p.wrow + (co % 32) * 8;
             for (int ci = 0; ci < C; ++ci)
-                for (int t = 0; t < T; ++t) {
-                    uint16_t *g = blk + ((size_t)(ci / 8) * T + t) * 512 + ci % 8;
-                    split_f16(get(co, ci, t), e, g[0], g[256]);
-                }
+                for (int t = 0; t < T; ++t)
+                    split_bf16(get(co, ci, t), blk + ((size_t)(ci / 8) * T + t) * 768 + ci % 8, 256);
         }
     });
     return p;
@@ -423,35 +441,6 @@ Packed pack_tail(Arena &A, int C, const float *w)
         }
     }
     return p;
-}
-
-// v as three bf16 parts, out[0], out[stride] and out[2 stride] (split.h): each
-// the nearest to what the ones before leave, the first towards zero where the
-// nearest would be infinite; infinities and NaNs whole in the third.
-void split_bf16(float v, uint16_t *out, size_t stride)
-{
-    auto bits = [](float x) {
-        uint32_t u;
-        std::memcpy(&u, &x, 4);
-        return u;
-    };
-    auto value = [](uint32_t u) {
-        float x;
-        std::memcpy(&x, &u, 4);
-        return x;
-    };
-    uint32_t u = bits(v);
-    if ((u & 0x7fffffff) >= 0x7f800000) {
-        out[0] = out[stride] = 0;
-        out[2 * stride] = (uint16_t)(u >> 16 | ((u & 0x7fffff) ? 0x40 : 0));
-        return;
-    }
-    for (int i = 0; i < 3; ++i, out += stride) {
-        uint32_t r = (u + 0x7fff + (u >> 16 & 1)) & 0xffff0000;  // to nearest, ties to even
-        if ((r & 0x7fffffff) == 0x7f800000) r = u & 0xffff0000;
-        *out = (uint16_t)(r >> 16);
-        u = bits(value(u) - value(r));
-    }
 }
 
 // Pointwise weights [M][C] for the kernels in three bf16 parts: [32 rows][group
