@@ -265,26 +265,25 @@ LAMA_EDGE_KERNEL(lama_convt_rows_q, up_body, 8, 16)
 
 // model.1: 7x7, reflect pad 3, at most 4 -> 64 channels, BN + ReLU, on the same
 // products.  K = 7 rows x 8 columns (the eighth zero) x 4 channels is 14 steps
-// of 16, whose weights, 112 registers a lane, are loaded once: a workgroup
+// of 16, whose weights, 168 registers a lane, are loaded once: a workgroup
 // walks tiles of 4 x 32 pixels, blockIdx.x, + gridDim.x, ...  Wave (wm, wn) owns
 // 32 channels and two tile rows.  A tile's input patch, loaded during the tile
-// before, is split with a scale of its own and stored as [part][pixel][4
-// channels] halves, so that lane group g's operand of a step, columns x + 4 s +
+// before, is split and stored as [part][pixel][4 channels], so that lane group g's operand of a step, columns x + 4 s +
 // 2 g and the next one, is two adjacent 8-byte words; two buffers, one barrier
 // a tile.
 //
-// What bounds it: the stores (2048x2048: 1.07 GB, 222 us at a copy's rate), not
-// fully hidden behind the next tile with two workgroups on a CU.  F32 MFMAs ->
-// split, us: 512x512 67 -> 26, 2048x2048 1020 -> 413.
+// What bounds it: the MFMAs (168 a tile and wave, 287 us of them at 2048x2048)
+// and the stores (1.07 GB, 222 us at a copy's rate), half hidden behind each
+// other.  F32 MFMAs / here, us: 512x512 67 / 48, 2048x2048 1020 / 621.
 namespace {
-constexpr int HR = 4, HC = 32, HPR = HR + 6, HPC = HC + 6, HST = 40, HPART = HPR * HST;  // LDS in h4
+constexpr int HR = 4, HC = 32, HPR = HR + 6, HPC = HC + 6, HST = 40, HPART = HPR * HST;  // LDS in b4
 constexpr int HNP = HPR * HPC, HPER = (HNP + LAMA_NT - 1) / LAMA_NT, HSTEPS = 14;
 }  // namespace
 extern "C" __global__ void __launch_bounds__(LAMA_NT) __attribute__((amdgpu_waves_per_eu(2)))
 lama_conv7x7r(LAMA_CONV_PARAMS)
 {
-    __shared__ __attribute__((aligned(16))) h4 xs[2 * 2 * HPART];
-    __shared__ float slot[12], epl[256];
+    __shared__ __attribute__((aligned(16))) b4 xs[2 * 3 * HPART];
+    __shared__ float epl[192];
     LAMA_STAMP_BEGIN;
     const ConvProblem P = probs[0];
     const ConvSeg &sg = P.s0;
@@ -311,129 +310,89 @@ lama_conv7x7r(LAMA_CONV_PARAMS)
             }
         }
     };
-    auto publish = [&](float *to, bool finite) {
-        float m = 0.f;
+    // tile number i of this workgroup, held in d, into its buffer
+    auto stage = [&](auto any, int i) {
+        b4 *const to = xs + (i & 1) * 3 * HPART;
+        float check = 0.f;
 #pragma unroll
-        for (int it = 0; it < HPER; ++it)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float a = fabsf(d[it][e]);
-                // as bits: a NaN counts as more than an infinity
-                m = finite ? fmaxf(m, a < __builtin_inff() ? a : 0.f)
-                           : __uint_as_float(max(__float_as_uint(m), __float_as_uint(a)));
-            }
-        m = wave_max(m);
-        if (lane == 0) to[wave] = m;
-    };
-    auto agreed = [&](const float *from) {
-        unsigned m = 0;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) m = max(m, __float_as_uint(from[w]));
-        return __uint_as_float((unsigned)__builtin_amdgcn_readfirstlane((int)m));
-    };
-    // tile number i of this workgroup, held in d, into its buffer; returns its scale's exponent
-    auto stage = [&](int i) {
-        float m = agreed(slot + 4 * (i & 1));
-        const bool inf = !(m < __builtin_inff());
-        if (inf) {  // the scale is that of the finite values
-            publish(slot + 8, true);
-            __syncthreads();
-            m = agreed(slot + 8);
+        for (int it = 0; it < HPER; ++it) {
+            const int pix = tid + it * LAMA_NT, r = pix / HPC, c = pix - r * HPC;
+            if (HNP % LAMA_NT && it == HPER - 1 && pix >= HNP) break;
+            b4 *p = to + r * HST + c;
+            check += split3<decltype(any)::value>(d[it], p[0], p[HPART], p[2 * HPART]);
         }
-        const int k = split_exp(SPLIT_K_START, m, 0);
-        const float s = pow2f(k);
-        h4 *const to = xs + (i & 1) * 2 * HPART;
-        auto store = [&](auto inf_) {
-#pragma unroll
-            for (int it = 0; it < HPER; ++it) {
-                const int pix = tid + it * LAMA_NT, r = pix / HPC, c = pix - r * HPC;
-                if (HNP % LAMA_NT && it == HPER - 1 && pix >= HNP) break;
-                h4 hi, lo;
-                split_n<decltype(inf_)::value>(d[it], s, hi, lo);
-                to[r * HST + c] = hi;
-                to[HPART + r * HST + c] = lo;
-            }
-        };
-        if (inf)
-            store(std::true_type{});
-        else
-            store(std::false_type{});
-        return k;
+        return check;
+    };
+    auto stage_any = [&](int i) {
+        if (split3_again(stage(std::false_type{}, i))) stage(std::true_type{}, i);
     };
     load(t);
-    // weights: [wm][step 2 ky + s][part][g][32][2 columns x 4 channels] halves
-    h8 wh[HSTEPS], wl[HSTEPS];
+    // weights: [wm][step 2 ky + s][part][g][32][2 columns x 4 channels]
+    b8 w0[HSTEPS], w1[HSTEPS], w2[HSTEPS];
     {
-        const LAMA_GLOBAL float *p = gp(sg.wt) + (long)min(wm, (P.M - 1) >> 5) * (HSTEPS * 512) + g * 128 + j * 4;
+        const LAMA_GLOBAL float *p = gp(sg.wt) + (long)min(wm, (P.M - 1) >> 5) * (HSTEPS * 768) + g * 128 + j * 4;
 #pragma unroll
         for (int st = 0; st < HSTEPS; ++st) {
-            wh[st] = *reinterpret_cast<const LAMA_GLOBAL h8 *>(p + st * 512);
-            wl[st] = *reinterpret_cast<const LAMA_GLOBAL h8 *>(p + st * 512 + 256);
+            w0[st] = *reinterpret_cast<const LAMA_GLOBAL b8 *>(p + st * 768);
+            w1[st] = *reinterpret_cast<const LAMA_GLOBAL b8 *>(p + st * 768 + 256);
+            w2[st] = *reinterpret_cast<const LAMA_GLOBAL b8 *>(p + st * 768 + 512);
         }
     }
-    {
+    if (tid < 192) {
         const int ec = min(tid & 63, P.M - 1);
         epl[tid] = tid < 64    ? (P.bias ? gp(P.bias)[ec] : 0.f)
                    : tid < 128 ? (P.scale ? gp(P.scale)[ec] : 1.f)
-                   : tid < 192 ? (P.scale ? gp(P.shift)[ec] : 0.f)
-                               : gp(sg.wsc)[ec];
+                               : (P.scale ? gp(P.shift)[ec] : 0.f);
     }
     // columns past the patch meet zero weights: zeros
-    for (int i = tid; i < 4 * HPR * (HST - HPC); i += LAMA_NT)
-        xs[i / (HST - HPC) * HST + HPC + i % (HST - HPC)] = h4{};
-    publish(slot, false);
-    __syncthreads();
-    int k = stage(0);
+    for (int i = tid; i < 6 * HPR * (HST - HPC); i += LAMA_NT)
+        xs[i / (HST - HPC) * HST + HPC + i % (HST - HPC)] = b4{};
+    stage_any(0);
     const int step = gridDim.x;
     load(min(t + step, ntiles - 1));  // past the last tile: that one again
-    publish(slot + 4, false);
     const int row0 = wm * 32 + 4 * g;  // register r: channel row0 + 8 (r / 4) + r % 4
     for (int i = 0;; ++i) {
         __syncthreads();
-        const int kn = t + step < ntiles ? stage(i + 1) : k;
+        if (t + step < ntiles) stage_any(i + 1);
         load(min(t + 2 * step, ntiles - 1));
         f32x16 acc[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[h][r] = 0.f;
-        const h4 *const rd = xs + (i & 1) * 2 * HPART + 2 * wn * HST + j + 2 * g;
-        h8 xh[2][2], xl[2][2];
-        auto read = [&](int st) {
+        const b4 *const rd = xs + (i & 1) * 3 * HPART + 2 * wn * HST + j + 2 * g;
+        b8 x[2][3];
+        auto read = [&](int u) {  // step u / 2 of tile row u % 2
+            const int st = u >> 1;
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const h4 *p = rd + (h + st / 2) * HST + 4 * (st & 1);
-                xh[st & 1][h] = __builtin_shufflevector(p[0], p[1], 0, 1, 2, 3, 4, 5, 6, 7);
-                xl[st & 1][h] = __builtin_shufflevector(p[HPART], p[HPART + 1], 0, 1, 2, 3, 4, 5, 6, 7);
+            for (int part = 0; part < 3; ++part) {
+                const b4 *p = rd + part * HPART + ((u & 1) + st / 2) * HST + 4 * (st & 1);
+                x[u & 1][part] = __builtin_shufflevector(p[0], p[1], 0, 1, 2, 3, 4, 5, 6, 7);
             }
         };
         read(0);
 #pragma unroll
-        for (int st = 0; st < HSTEPS; ++st) {
-            if (st + 1 < HSTEPS) read(st + 1);
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-                acc[h] = mfma_split(wh[st], wl[st], xh[st & 1][h], xl[st & 1][h], acc[h]);
+        for (int u = 0; u < 2 * HSTEPS; ++u) {
+            if (u + 1 < 2 * HSTEPS) read(u + 1);
+            const auto &v = x[u & 1];
+            mfma_split3(w0[u >> 1], w1[u >> 1], w2[u >> 1], v[0], v[1], v[2], acc[u & 1], acc[u & 1]);
         }
-        const float u = pow2f(-k);  // |k| <= 100
-        const int y0 = (t / tiles_x) * HR + 2 * wn, x = (t % tiles_x) * HC + j;
+        const int y0 = (t / tiles_x) * HR + 2 * wn, ox = (t % tiles_x) * HC + j;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            if (y0 + h >= P.OH || x >= P.OW) continue;
-            LAMA_GLOBAL float *out = gp(P.out) + (long)row0 * P.out_cstride + (long)(y0 + h) * P.outW + x;
+            if (y0 + h >= P.OH || ox >= P.OW) continue;
+            LAMA_GLOBAL float *out = gp(P.out) + (long)row0 * P.out_cstride + (long)(y0 + h) * P.outW + ox;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int rr = 8 * (r >> 2) + (r & 3), cl = row0 + rr;
                 if (cl >= P.M) continue;
-                float v = acc[h][r] * epl[192 + cl] * u + epl[cl];
+                float v = acc[h][r] + epl[cl];
                 v = v * epl[64 + cl] + epl[128 + cl];
                 out[(long)rr * P.out_cstride] = P.relu ? fmaxf(v, 0.f) : v;
             }
         }
         t += step;
         if (t >= ntiles) break;
-        publish(slot + 4 * (i & 1), false);
-        k = kn;
     }
     LAMA_STAMP_END;
 }

@@ -379,9 +379,8 @@ Packed pack_taps(Arena &A, int M, int C, int T, const Get &get)
 }
 
 // The head's 7x7 weights (at most 64 x 4 channels) for lama_conv7x7r: [32 rows]
-// [step 2 ky + kx / 4][hi, lo][kx % 4 / 2][32][kx % 2][4 channels] halves, the
-// eighth column, channels past C and rows past M zero; the row scales beside
-// them.
+// [step 2 ky + kx / 4][part][kx % 4 / 2][32][kx % 2][4 channels], the eighth
+// column, channels past C and rows past M zero.
 template <class Get>
 Packed pack_head(Arena &A, int M, int C, const Get &get)
 {
@@ -391,24 +390,16 @@ Packed pack_head(Arena &A, int M, int C, const Get &get)
     p.T = 49;
     p.KC = 4;
     p.nchunk = 1;
-    p.wrow = 14 * 16;
+    p.wrow = 14 * 24;
     p.off = A.add((size_t)((M + 31) / 32) * 32 * p.wrow);
-    p.ws = A.add(M);
     uint16_t *d = reinterpret_cast<uint16_t *>(A.at(p.off));
-    for (int co = 0; co < M; ++co) {
-        float most = 0;
-        for (int i = 0; i < C * 49; ++i) {
-            const float x = get(co, i / 49, i % 49);
-            if (std::isfinite(x)) most = std::max(most, std::fabs(x));
-        }
-        const int e = split_row_exp(most);
-        A.at(p.ws)[co] = std::ldexp(1.f, -e);
+    for (int co = 0; co < M; ++co)
         for (int i = 0; i < C * 49; ++i) {
             const int ci = i / 49, ky = i % 49 / 7, kx = i % 7;
-            uint16_t *g = d + ((size_t)(co / 32) * 14 + 2 * ky + kx / 4) * 1024 + kx % 4 / 2 * 256 + co % 32 * 8 + kx % 2 * 4 + ci;
-            split_f16(get(co, ci, i % 49), e, g[0], g[512]);
+            split_bf16(get(co, ci, i % 49),
+                       d + ((size_t)(co / 32) * 14 + 2 * ky + kx / 4) * 1536 + kx % 4 / 2 * 256 + co % 32 * 8 + kx % 2 * 4 + ci,
+                       512);
         }
-    }
     return p;
 }
 
