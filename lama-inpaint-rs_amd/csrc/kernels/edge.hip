@@ -344,9 +344,6 @@ lama_conv7x7r(LAMA_CONV_PARAMS)
                    : tid < 128 ? (P.scale ? gp(P.scale)[ec] : 1.f)
                                : (P.scale ? gp(P.shift)[ec] : 0.f);
     }
-    // columns past the patch meet zero weights: zeros
-    for (int i = tid; i < 6 * HPR * (HST - HPC); i += LAMA_NT)
-        xs[i / (HST - HPC) * HST + HPC + i % (HST - HPC)] = b4{};
     stage_any(0);
     const int step = gridDim.x;
     load(min(t + step, ntiles - 1));  // past the last tile: that one again
@@ -367,7 +364,10 @@ lama_conv7x7r(LAMA_CONV_PARAMS)
 #pragma unroll
             for (int part = 0; part < 3; ++part) {
                 const b4 *p = rd + part * HPART + ((u & 1) + st / 2) * HST + 4 * (st & 1);
-                x[u & 1][part] = __builtin_shufflevector(p[0], p[1], 0, 1, 2, 3, 4, 5, 6, 7);
+                // the eighth column lies outside the window: zeros, as the zero
+                // weights it meets would make NaN of an infinity
+                const b4 second = (st & 1) && g ? b4{} : p[1];
+                x[u & 1][part] = __builtin_shufflevector(p[0], second, 0, 1, 2, 3, 4, 5, 6, 7);
             }
         };
         read(0);
