@@ -78,7 +78,7 @@ static inline constexpr int lama_convt_kc(int phase)
 #endif
 // output tile of the 7x7 tail kernel (rows x columns): 64 columns of partial
 // sums less the six that only feed their neighbours
-#define LAMA_TAIL_ROWS 8
+#define LAMA_TAIL_ROWS 6
 #define LAMA_TAIL_COLS 58
 
 #ifdef __HIP_DEVICE_COMPILE__
@@ -267,8 +267,7 @@ struct FinalizeArgs {
 // mask, h x w with h <= H, w <= W, and writes the 8-bit composite.
 struct TailArgs {
     const float *src;  // [Cin][H][W]
-    const float *wt;   // halves, by 16-channel chunk and ky (pack_tail)
-    const float *wsc;  // [32]: 2^-e of every row 7 co + kx, e its weights' scale
+    const float *wt;   // bf16 parts, by 16-channel chunk and ky (pack_tail)
     const float *bias; // [3]
     float *out;        // [3][H][W]
     int Cin, H, W;

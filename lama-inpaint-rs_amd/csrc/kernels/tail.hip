@@ -1,24 +1,25 @@
 // model.34 + model.35: 7x7 convolution 64 -> 3 over the ReflectionPad2d(3)
-// plane, with bias, then sigmoid (cpu.rs:531-534, 384-388), on split f16
-// products (split.h).
+// plane, with bias, then sigmoid (cpu.rs:531-534, 384-388), on three bf16 parts
+// (split.h).
 //
 // Three output channels alone would leave 90% of an MFMA's rows empty, so the
 // rows are (channel, kx), 21 of 32: with
 //     p[co, kx][y][x'] = sum over (ci, ky) of w[co][ci][ky][kx] in[ci][y + ky][x']
 // an output is the sum of seven neighbours, out[co][y][x] = sum over kx of
-// p[co, kx][y][x + kx], taken from LDS at the end.  A workgroup computes p for 8
-// rows x 64 columns, hence 8 x 58 outputs; wave (rh, ch) owns four rows of 32
-// columns, four accumulators.  K is walked in chunks of 16 channels: a chunk's
-// 14 x 64 input patch, loaded into registers during the chunk before, is scaled,
-// split and stored as [part][8-channel group][pixel][8] halves, so that an MFMA
-// operand is one 16-byte read a lane; one input row's operand serves up to four
-// output rows (ky = 0..6), whose weights the wave holds for the chunk and
-// replaces as soon as their last row is done.
+// p[co, kx][y][x + kx], taken from LDS at the end.  A workgroup computes p for 6
+// rows x 64 columns, hence 6 x 58 outputs; wave (rh, ch) owns three rows of 32
+// columns, three accumulators.  K is walked in chunks of 16 channels: a chunk's
+// 12 x 64 input patch, loaded into registers during the chunk before, is split
+// and stored as [part][8-channel group][pixel][8], so that an MFMA operand is one
+// 16-byte read a lane; one input row's operand serves up to three output rows
+// (ky = 0..6), whose weights the wave holds for the chunk and replaces as soon as
+// their last row is done.  Six rows, not eight: 72 KB of LDS, two workgroups a CU
+// (84 KB with eight).
 //
-// What bounds it: staging (14 x 64 pixels read for 8 x 58 outputs) and the
-// MFMAs about equally; the input alone is 1.07 GB at 2048x2048, 222 us at a
-// copy's rate.  F32 FMAs on the vector units -> split, us: 512x512 76 -> 38,
-// 2048x2048 1180 -> 458.
+// What bounds it: the MFMAs and staging (12 x 64 pixels read for 6 x 58 outputs)
+// about equally; the input alone is 1.07 GB at 2048x2048, 222 us at a copy's
+// rate.  F32 FMAs on the vector units / here, us: 512x512 76 / 55, 2048x2048
+// 1180 / 713.
 #include <hip/hip_runtime.h>
 
 #include "common.h"
@@ -28,10 +29,11 @@ namespace {
 constexpr int TROWS = LAMA_TAIL_ROWS, TCOLS = LAMA_TAIL_COLS;  // outputs
 constexpr int TPR = TROWS + 6, TPC = TCOLS + 6, TNP = TPR * TPC;  // patch
 constexpr int THALF = LAMA_NT / 2, TPER = TNP / THALF;         // pixels a thread stages, of one channel group
-constexpr int TGS = TNP, TPS = 2 * TGS;                        // group and part strides, h8
-static_assert(THALF == 2 * TPC && TROWS == 8 && TPC == 64, "four waves of 4 rows x 32 columns");
+constexpr int TRW = TROWS / 2;                                 // rows a wave owns
+constexpr int TGS = TNP, TPS = 2 * TGS;                        // group and part strides, b8
+static_assert(THALF == 2 * TPC && TROWS % 2 == 0 && TROWS <= 8 && TPC == 64, "four waves of TRW rows x 32 columns");
 static_assert(TNP % THALF == 0, "whole staging rounds");
-static_assert(TROWS * 21 * TPC * 4 <= 2 * TPS * 16, "the sums over (ci, ky) fit in the patch buffer");
+static_assert(TROWS * 21 * TPC * 4 <= 3 * TPS * 16, "the sums over (ci, ky) fit in the patch buffer");
 
 }  // namespace
 
@@ -55,8 +57,7 @@ __device__ __forceinline__ uint8_t composite_u8(float v)
 template <bool U8>
 __device__ __forceinline__ void tail_body(const TailArgs *__restrict__ args, int h, int w)
 {
-    __shared__ h8 xs[2 * TPS];
-    __shared__ float slot[8];
+    __shared__ b8 xs[3 * TPS];
     const TailArgs A = *args;
     const int H = A.H, W = A.W, nc = A.Cin, n = (nc + 15) / 16;
     const int tiles_x = (W + TCOLS - 1) / TCOLS;
@@ -83,22 +84,32 @@ __device__ __forceinline__ void tail_body(const TailArgs *__restrict__ args, int
         }
     };
     load(0);
-    // weights: [16-channel chunk][ky][part][8-channel group][32 rows 7 co + kx][8] halves
-    h8 wh[7], wl[7];
+    // weights: [16-channel chunk][ky][part][8-channel group][32 rows 7 co + kx][8]
+    b8 w0[7], w1[7], w2[7];
     auto load_w = [&](int ky, int ck) {
-        const LAMA_GLOBAL float *p = gp(A.wt) + (ck * 7 + ky) * 512 + lane * 4;
-        wh[ky] = *reinterpret_cast<const LAMA_GLOBAL h8 *>(p);
-        wl[ky] = *reinterpret_cast<const LAMA_GLOBAL h8 *>(p + 256);
+        const LAMA_GLOBAL float *p = gp(A.wt) + (ck * 7 + ky) * 768 + lane * 4;
+        w0[ky] = *reinterpret_cast<const LAMA_GLOBAL b8 *>(p);
+        w1[ky] = *reinterpret_cast<const LAMA_GLOBAL b8 *>(p + 256);
+        w2[ky] = *reinterpret_cast<const LAMA_GLOBAL b8 *>(p + 512);
     };
 #pragma unroll
     for (int ky = 0; ky < 7; ++ky) load_w(ky, 0);
-    f32x16 acc[4];
+    f32x16 acc[TRW];
 #pragma unroll
-    for (int y = 0; y < 4; ++y)
+    for (int y = 0; y < TRW; ++y)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[y][r] = 0.f;
-    const h8 *const rd = xs + g * TGS + rh * 4 * TPC + ch * 32 + j;
-    int k = SPLIT_K_START;
+    const b8 *const rd = xs + g * TGS + rh * TRW * TPC + ch * 32 + j;
+    auto stage = [&](auto any) {
+        b8 *const to = xs + ig * TGS + it0;
+        float check = 0.f;
+#pragma unroll
+        for (int it = 0; it < TPER; ++it) {
+            b8 *p = to + it * THALF;
+            check += split3<decltype(any)::value>(d[it], p[0], p[TPS], p[2 * TPS]);
+        }
+        return check;
+    };
     for (int ck = 0; ck < n; ++ck) {
         if ((ck + 1) * 16 > nc) {
 #pragma unroll
@@ -107,77 +118,31 @@ __device__ __forceinline__ void tail_body(const TailArgs *__restrict__ args, int
 #pragma unroll
                     for (int it = 0; it < TPER; ++it) d[it][e] = 0.f;
         }
-        auto agree = [&](bool finite, float *at) {  // the workgroup's largest magnitude
-            float m = 0.f;
-#pragma unroll
-            for (int it = 0; it < TPER; ++it)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float a = fabsf(d[it][e]);
-                    // as bits: a NaN counts as more than an infinity
-                    m = finite ? fmaxf(m, a < __builtin_inff() ? a : 0.f)
-                               : __uint_as_float(max(__float_as_uint(m), __float_as_uint(a)));
-                }
-            m = wave_max(m);
-            if (lane == 0) at[wave] = m;
-            __syncthreads();  // and every wave is done with the last chunk's operands
-            unsigned v = 0;
-#pragma unroll
-            for (int w = 0; w < 4; ++w) v = max(v, __float_as_uint(at[w]));
-            return __uint_as_float((unsigned)__builtin_amdgcn_readfirstlane((int)v));
-        };
-        float m = agree(false, slot);
-        const bool inf = !(m < __builtin_inff());
-        if (inf) m = agree(true, slot + 4);  // the scale is that of the finite values
-        const int kn = split_exp(k, m, 0);
-        if (kn != k) {
-            if (ck > 0) {
-                const float f = pow2f(max(kn - k, -126));
-#pragma unroll
-                for (int y = 0; y < 4; ++y)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[y][r] *= f;
-            }
-            k = kn;
-        }
-        const float s = pow2f(k);
-        auto store = [&](auto inf_) {
-            h8 *const to = xs + ig * TGS + it0;
-#pragma unroll
-            for (int it = 0; it < TPER; ++it) {
-                h8 hi, lo;
-                split_n<decltype(inf_)::value>(d[it], s, hi, lo);
-                to[it * THALF] = hi;
-                to[it * THALF + TPS] = lo;
-            }
-        };
-        if (inf)
-            store(std::true_type{});
-        else
-            store(std::false_type{});
+        if (ck > 0) __syncthreads();  // every wave is done with the last chunk's operands
+        if (split3_again(stage(std::false_type{}))) stage(std::true_type{});
         load(min(ck + 1, n - 1));  // unconditional: the waits then count exactly
         __syncthreads();
         // each input row's operand reads are issued before the row before it
-        h8 xh[2], xl[2];
+        b8 x[2][3];
         auto read = [&](int r) {
-            xh[r & 1] = rd[r * TPC];
-            xl[r & 1] = rd[r * TPC + TPS];
+#pragma unroll
+            for (int part = 0; part < 3; ++part) x[r & 1][part] = rd[r * TPC + part * TPS];
         };
         read(0);
 #pragma unroll
-        for (int r = 0; r < 10; ++r) {
-            if (r + 1 < 10) read(r + 1);
-            // the three products of up to four rows in turn: no MFMA waits for the one before it
+        for (int r = 0; r < TRW + 6; ++r) {
+            if (r + 1 < TRW + 6) read(r + 1);
+            // the six products of the rows in turn: no MFMA waits for the one before it
 #pragma unroll
-            for (int part = 0; part < 3; ++part)
+            for (int i = 0; i < 6; ++i)
 #pragma unroll
-                for (int y = 0; y < 4; ++y) {
+                for (int y = 0; y < TRW; ++y) {
                     const int ky = r - y;
                     if (ky < 0 || ky > 6) continue;
-                    acc[y] = __builtin_amdgcn_mfma_f32_32x32x16_f16(part == 0 ? wl[ky] : wh[ky],
-                                                                    part == 1 ? xl[r & 1] : xh[r & 1], acc[y], 0, 0, 0);
+                    acc[y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        SPLIT3_A[i] == 0 ? w0[ky] : SPLIT3_A[i] == 1 ? w1[ky] : w2[ky], x[r & 1][SPLIT3_X[i]], acc[y], 0, 0, 0);
                 }
-            if (r >= 3) load_w(r - 3, min(ck + 1, n - 1));
+            if (r >= TRW - 1) load_w(r - (TRW - 1), min(ck + 1, n - 1));
             // keep the load here: the scheduler would otherwise sink it below
             // the chunk's last MFMA
             __builtin_amdgcn_sched_barrier(0);
@@ -186,18 +151,16 @@ __device__ __forceinline__ void tail_body(const TailArgs *__restrict__ args, int
     __syncthreads();  // every wave is done with the operands
     // p[row][7 co + kx][column], in the patch buffer; register r: row 8 (r / 4) + 4 g + r % 4
     float *const ps = reinterpret_cast<float *>(xs);
-    const float u = pow2f(-k);  // |k| <= 100 once a chunk has been taken
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int i = 8 * (r >> 2) + 4 * g + (r & 3);
         if (i >= 21) continue;
-        const float sc = gp(A.wsc)[i];
 #pragma unroll
-        for (int y = 0; y < 4; ++y) ps[((rh * 4 + y) * 21 + i) * TPC + ch * 32 + j] = acc[y][r] * sc * u;
+        for (int y = 0; y < TRW; ++y) ps[((rh * TRW + y) * 21 + i) * TPC + ch * 32 + j] = acc[y][r];
     }
     __syncthreads();
     const int oy = oy0 + (tid >> 5);
-    if (oy >= H) return;
+    if ((tid >> 5) >= TROWS || oy >= H) return;
     float bias[3];
 #pragma unroll
     for (int co = 0; co < 3; ++co) bias[co] = gp(A.bias)[co];

@@ -403,9 +403,9 @@ Packed pack_head(Arena &A, int M, int C, const Get &get)
     return p;
 }
 
-// The tail's weights w [3][C][7][7] for lama_tail: [16-channel chunk][ky][hi, lo]
-// [group of 8 channels][32 rows 7 co + kx][8] halves, rows past 20 and channels
-// past C zero; the 32 row scales beside them.
+// The tail's weights w [3][C][7][7] for lama_tail: [16-channel chunk][ky][part]
+// [group of 8 channels][32 rows 7 co + kx][8], rows past 20 and channels past C
+// zero.
 Packed pack_tail(Arena &A, int C, const float *w)
 {
     Packed p;
@@ -414,23 +414,14 @@ Packed pack_tail(Arena &A, int C, const float *w)
     p.T = 7;
     p.KC = 16;
     p.nchunk = (C + 15) / 16;
-    p.off = A.add((size_t)p.nchunk * 7 * 512);
-    p.ws = A.add(32);
+    p.off = A.add((size_t)p.nchunk * 7 * 768);
     uint16_t *d = reinterpret_cast<uint16_t *>(A.at(p.off));
-    for (int row = 0; row < 21; ++row) {
-        const int co = row / 7, kx = row % 7;
-        auto get = [&](int i) { return w[((size_t)co * C + i / 7) * 49 + i % 7 * 7 + kx]; };  // i: channel, ky
-        float most = 0;
-        for (int i = 0; i < C * 7; ++i)
-            if (std::isfinite(get(i))) most = std::max(most, std::fabs(get(i)));
-        const int e = split_row_exp(most);
-        A.at(p.ws)[row] = std::ldexp(1.f, -e);
-        for (int i = 0; i < C * 7; ++i) {
+    for (int row = 0; row < 21; ++row)
+        for (int i = 0; i < C * 7; ++i) {  // channel, ky
             const int ci = i / 7;
-            uint16_t *g = d + ((size_t)(ci / 16) * 7 + i % 7) * 1024 + ci % 16 / 8 * 256 + row * 8 + ci % 8;
-            split_f16(get(i), e, g[0], g[512]);
+            split_bf16(w[((size_t)(row / 7) * C + ci) * 49 + i % 7 * 7 + row % 7],
+                       d + ((size_t)(ci / 16) * 7 + i % 7) * 1536 + ci % 16 / 8 * 256 + row * 8 + ci % 8, 512);
         }
-    }
     return p;
 }
 
@@ -1918,7 +1909,6 @@ bool Engine::build_plan(Plan &p, void *arena, std::string &err)
     TailArgs ta{};
     ta.src = a1;
     ta.wt = wp(tail_.off);
-    ta.wsc = wp(tail_.ws);
     ta.bias = wp(tail_b_);
     ta.out = out;
     ta.Cin = 64;
@@ -3149,7 +3139,6 @@ bool Engine::op_tail(const float *x, int cin, int h, int w, const float *wt, con
     TailArgs a{};
     a.src = dx;
     a.wt = dw + pk.off;
-    a.wsc = dw + pk.ws;
     a.bias = db;
     a.out = dout;
     a.Cin = cin;
