@@ -148,13 +148,11 @@ __device__ __forceinline__ int reflect1(int i, int n)
 // bottleneck planes are padded to a multiple of 4 floats so that every plane
 // is 16-byte aligned); `wt` points at row 0 of the packed weights
 // [M][nchunk][taps][KC] (KC input channels per chunk, zero-padded).
-// Split-product kernels (split.h): `wt` holds f16 halves in their operand
-// order, wrow floats of room a row, nchunk counts 16-channel steps (pointwise)
-// and `wsc` is 2^-e of every output channel, e its weights' scale.
+// Kernels on three bf16 parts (split.h): `wt` holds the parts in operand
+// order, wrow floats of room a row; nchunk counts 16-channel steps (pointwise).
 struct ConvSeg {
     const float *src;
     const float *wt;
-    const float *wsc;
     int C, IH, IW;
     int nchunk;
     int wrow;  // floats per packed weight row = nchunk * taps * KC
@@ -282,11 +280,11 @@ struct TailArgs {
 // src0 [M][C0][9], the rest from src1 [M][C - C0][9] (the FFC's local GEMM
 // concatenates l2l and g2l along K).  kind 4: the F(4,3) layout of
 // lama_conv3x3w4*; kind 42: the F(2x4, 3x3) layout of lama_conv3x3w42.
-// dst is pre-zeroed (rows past M, channels past C stay zero).  kind 4 is a
-// split pack (split.h): halves scaled by 2^e of their row, 2^-e into wsc.
+// Both hold three bf16 parts of every value (split.h).  dst is pre-zeroed (rows
+// past M, channels past C stay zero).
 struct WinoPackJob {
     const float *src0, *src1;
-    float *dst, *wsc;
+    float *dst;
     int M, C, C0, nchunk, kind;
     int pad_;
 };

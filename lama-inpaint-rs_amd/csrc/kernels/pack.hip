@@ -10,7 +10,7 @@
 // on the host: this code object is built with -ffp-contract=fast, under
 // which the backend fuses a multiply and an add into one FMA whatever the
 // source says, so each product passes through an empty asm statement that
-// hides it from that combine.  The packed floats are then identical.
+// hides it from that combine.  The packed parts are then identical.
 //
 // F(4,3) along x: U_u = sum over kx of G[u][kx] w[ky][kx], G for the points
 // 0, 1, -1, 2, -2, infinity.  F(2x4, 3x3): U(vy, u) = sum over kx of
@@ -31,6 +31,16 @@ __device__ __forceinline__ double dot3(double a, double x, double b, double y, d
     return p + q + r;
 }
 
+// the three parts of x (split.h), 256 apart
+__device__ __forceinline__ void put_parts(LAMA_GLOBAL __bf16 *at, float x)
+{
+    const float v[2] = {x, 0.f};
+    b2 p[3];
+    split3<true>(v, p[0], p[1], p[2]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) at[256 * i] = p[i][0];
+}
+
 // U_u of kernel row ky, u < 6, ky < 3, of one channel pair
 __device__ __forceinline__ void transform_w43(const double (&g)[9], float (&v)[6][3])
 {
@@ -44,22 +54,15 @@ __device__ __forceinline__ void transform_w43(const double (&g)[9], float (&v)[6
 }
 
 // [64 rows][8-channel group][wave (wm, u / 3)][step ky * 3 + u % 3][part][32][8]
-__device__ __forceinline__ void pack_one_w43(const WinoPackJob &J, int co, int ci, float s, const float (&v)[6][3])
+__device__ __forceinline__ void pack_one_w43(const WinoPackJob &J, int co, int ci, const float (&v)[6][3])
 {
     const int mb = co / 64, wm = co % 64 / 32, j = co % 32;
-    LAMA_GLOBAL _Float16 *blk = reinterpret_cast<LAMA_GLOBAL _Float16 *>(gp(J.dst)) +
-                                ((long)mb * (J.nchunk / 2) + ci / 8) * 18432 + j * 8 + ci % 8;
+    LAMA_GLOBAL __bf16 *blk = reinterpret_cast<LAMA_GLOBAL __bf16 *>(gp(J.dst)) +
+                              ((long)mb * (J.nchunk / 2) + ci / 8) * 27648 + j * 8 + ci % 8;
 #pragma unroll
     for (int u = 0; u < 6; ++u)
 #pragma unroll
-        for (int ky = 0; ky < 3; ++ky) {
-            const float x[2] = {v[u][ky], 0.f};
-            h2 hi, lo;
-            split_n<true>(x, s, hi, lo);
-            const int at = ((wm * 2 + u / 3) * 9 + ky * 3 + u % 3) * 512;
-            blk[at] = hi[0];
-            blk[at + 256] = lo[0];
-        }
+        for (int ky = 0; ky < 3; ++ky) put_parts(blk + ((wm * 2 + u / 3) * 9 + ky * 3 + u % 3) * 768, v[u][ky]);
 }
 
 // U(vy, u), vy < 4, u < 6, of one channel pair
@@ -79,54 +82,13 @@ __device__ __forceinline__ void transform_w42(const double (&g)[9], float (&v)[4
 }
 
 // [64 rows][8-channel group][wave (wm, vy)][u][part][32][8]
-__device__ __forceinline__ void pack_one_w42(const WinoPackJob &J, int co, int ci, float s, const float (&v)[4][6])
+__device__ __forceinline__ void pack_one_w42(const WinoPackJob &J, int co, int ci, const float (&v)[4][6])
 {
     const int mb = co / 64, wm = co % 64 / 32, j = co % 32;
-    LAMA_GLOBAL _Float16 *blk = reinterpret_cast<LAMA_GLOBAL _Float16 *>(gp(J.dst)) +
-                                ((long)mb * (J.nchunk / 2) + ci / 8) * 24576 + wm * 12288 + j * 8 + ci % 8;
+    LAMA_GLOBAL __bf16 *blk = reinterpret_cast<LAMA_GLOBAL __bf16 *>(gp(J.dst)) +
+                              ((long)mb * (J.nchunk / 2) + ci / 8) * 36864 + wm * 18432 + j * 8 + ci % 8;
 #pragma unroll
-    for (int i = 0; i < 24; ++i) {
-        const float x[2] = {v[i / 6][i % 6], 0.f};
-        h2 hi, lo;
-        split_n<true>(x, s, hi, lo);
-        blk[i * 512] = hi[0];
-        blk[i * 512 + 256] = lo[0];
-    }
-}
-
-// One output channel's row: the largest of its N values sets its scale.
-template <class V, class T, class W>
-__device__ __forceinline__ void pack_row(const WinoPackJob &J, int co, float *slot, T transform, W write)
-{
-    V v;
-    constexpr int N = sizeof v / 4;
-    auto taps = [&](int ci) {
-        double g[9];
-        const LAMA_GLOBAL float *s = ci < J.C0 ? gp(J.src0) + ((long)co * J.C0 + ci) * 9
-                                               : gp(J.src1) + ((long)co * (J.C - J.C0) + (ci - J.C0)) * 9;
-#pragma unroll
-        for (int k = 0; k < 9; ++k) g[k] = (double)s[k];
-        transform(g, v);
-    };
-    float m = 0.f;
-    for (int ci = threadIdx.x; ci < J.C; ci += 256) {
-        taps(ci);
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            const float a = fabsf((&v[0][0])[i]);
-            m = fmaxf(m, a < __builtin_inff() ? a : 0.f);
-        }
-    }
-    m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) slot[threadIdx.x >> 6] = m;
-    __syncthreads();
-    m = fmaxf(fmaxf(slot[0], slot[1]), fmaxf(slot[2], slot[3]));
-    const int e = m > 0.f ? max(-100, min(100, 14 - exp2_of(m))) : 0;
-    if (threadIdx.x == 0) gp(J.wsc)[co] = pow2f(-e);
-    for (int ci = threadIdx.x; ci < J.C; ci += 256) {
-        taps(ci);
-        write(ci, pow2f(e), v);
-    }
+    for (int i = 0; i < 24; ++i) put_parts(blk + i * 768, v[i / 6][i % 6]);
 }
 
 }  // namespace
@@ -135,18 +97,23 @@ __device__ __forceinline__ void pack_row(const WinoPackJob &J, int co, float *sl
 // output channel's row; rows past the job's M have nothing to do.
 extern "C" __global__ void __launch_bounds__(256) lama_pack_wino(const WinoPackJob *__restrict__ jobs)
 {
-    __shared__ float slot[4];
     const WinoPackJob J = jobs[blockIdx.y];
     const int co = blockIdx.x;
     if (co >= J.M) return;  // whole workgroup
-    typedef float V43[6][3];
-    typedef float V42[4][6];
-    if (J.kind == 42)
-        pack_row<V42>(
-            J, co, slot, [](const double(&g)[9], V42 &v) { transform_w42(g, v); },
-            [&](int ci, float s, const V42 &v) { pack_one_w42(J, co, ci, s, v); });
-    else
-        pack_row<V43>(
-            J, co, slot, [](const double(&g)[9], V43 &v) { transform_w43(g, v); },
-            [&](int ci, float s, const V43 &v) { pack_one_w43(J, co, ci, s, v); });
+    for (int ci = threadIdx.x; ci < J.C; ci += 256) {
+        double g[9];
+        const LAMA_GLOBAL float *s = ci < J.C0 ? gp(J.src0) + ((long)co * J.C0 + ci) * 9
+                                               : gp(J.src1) + ((long)co * (J.C - J.C0) + (ci - J.C0)) * 9;
+#pragma unroll
+        for (int k = 0; k < 9; ++k) g[k] = (double)s[k];
+        if (J.kind == 42) {
+            float v[4][6];
+            transform_w42(g, v);
+            pack_one_w42(J, co, ci, v);
+        } else {
+            float v[6][3];
+            transform_w43(g, v);
+            pack_one_w43(J, co, ci, v);
+        }
+    }
 }

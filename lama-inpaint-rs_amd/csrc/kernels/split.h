@@ -105,80 +105,3 @@ __device__ __forceinline__ void mfma_split3(const b8 &a0, const b8 &a1, const b8
 }
 
 }  // namespace
-
-// Scaled f16 halves, x s = hi + lo: the kernels that still take these.
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-
-namespace {
-
-__device__ __forceinline__ float pow2f(int e) { return __uint_as_float((unsigned)(127 + e) << 23); }
-
-// floor(log2 m) of a finite m >= 0 (subnormals and 0: -127)
-__device__ __forceinline__ int exp2_of(float m) { return (int)(__float_as_uint(m) >> 23) - 127; }
-
-// The largest of the wave's 64 values (none negative; NaN above infinity), in
-// every lane.  Compared as bits: each step is then one DPP instruction.
-__device__ __forceinline__ float wave_max(float f)
-{
-    unsigned v = __float_as_uint(f);
-    auto step = [&](auto ctrl) {
-        // lanes without a source take 0
-        v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, 0xf, 0xf, false));
-    };
-    step(std::integral_constant<int, 0x111>{});  // row_shr:1
-    step(std::integral_constant<int, 0x112>{});
-    step(std::integral_constant<int, 0x114>{});
-    step(std::integral_constant<int, 0x118>{});
-    step(std::integral_constant<int, 0x142>{});  // row_bcast:15
-    step(std::integral_constant<int, 0x143>{});  // row_bcast:31: lane 63 holds the wave's
-    return __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)v, 63));
-}
-
-// The scale exponent a tile keeps: values of magnitude up to m (the largest
-// of the next chunk) must stay below 2^15 after `gain` further bits; k is
-// lowered to leave three bits of headroom when they would not.  k starts at
-// SPLIT_K_START and stays within +-100, so that 2^k and 2^-k are normal.
-constexpr int SPLIT_K_START = 127;
-__device__ __forceinline__ int split_exp(int k, float m, int gain)
-{
-    const int most = 14 - gain - exp2_of(m);
-    return k <= most ? k : max(-100, min(100, most - 3));
-}
-
-// hi and lo of N values times s, two at a time.  The pair of his passes
-// through an empty asm statement: the compiler otherwise converts each of them
-// a second time for the subtraction.  INF: some value may be infinite or NaN.
-template <bool INF, int N, class H>
-__device__ __forceinline__ void split_n(const float (&x)[N], float s, H &hi, H &lo)
-{
-#pragma unroll
-    for (int e = 0; e < N; e += 2) {
-        h2 a = {(_Float16)(x[e] * s), (_Float16)(x[e + 1] * s)};
-        asm("" : "+v"(a));
-        h2 b = {(_Float16)fmaf(x[e], s, -(float)a[0]), (_Float16)fmaf(x[e + 1], s, -(float)a[1])};
-        if constexpr (INF) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-                if (!(fabsf(x[e + i]) < __builtin_inff())) {
-                    a[i] = (_Float16)0.f;
-                    b[i] = (_Float16)x[e + i];
-                }
-        }
-        hi[e] = a[0];
-        hi[e + 1] = a[1];
-        lo[e] = b[0];
-        lo[e + 1] = b[1];
-    }
-}
-
-// c += a b as three MFMAs; the small products first.
-__device__ __forceinline__ f32x16 mfma_split(const h8 &ah, const h8 &al, const h8 &bh, const h8 &bl, f32x16 c)
-{
-    c = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh, c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl, c, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh, c, 0, 0, 0);
-}
-
-}  // namespace

@@ -1,5 +1,5 @@
 // FFC 3x3 convolutions (stride 1, reflect pad 1) as a two-dimensional
-// Winograd F(2x4, 3x3) on split f16 products (split.h): F(2,3) along y (points
+// Winograd F(2x4, 3x3) on three bf16 parts (split.h): F(2,3) along y (points
 // 0, 1, -1, infinity) times the F(4,3) of lama_conv3x3w4 along x.  An output
 // tile is 2 rows x 4 pixels, read from input rows r0..r3 x the six columns
 // d0..d5 of each:
@@ -18,22 +18,22 @@
 // block's 32 tiles).  K is walked in chunks of 16 channels through two LDS
 // buffers, one barrier a chunk: while the MFMAs of a chunk run, the next one,
 // in registers, is transformed, split and stored as [part][8-channel group]
-// [position][tile][8] halves, position by position between the MFMAs, and the
-// one after it is loaded.  A staging thread takes four channels of one tile
+// [position][tile][8], position by position between the MFMAs, and the one
+// after it is loaded.  A staging thread takes four channels of one tile
 // and one vy, so it combines two input rows before the x transform; d0 and d5
 // come from the neighbouring lanes (a tile row is a DPP row), so a row costs
 // one 16-byte load a lane and one for the halo columns.  Each wave loads its
-// own weights in operand order, three positions ahead.  In the epilogue every wave
+// own weights in operand order, two positions (12 MFMAs) ahead.  In the epilogue every wave
 // applies A_x^T to its six accumulators and parks the four pixels in LDS; each
 // wave then finishes four of the 16 register rows of its channel half, both
 // output rows, from the four y positions.
 //
-// What bounds it: the loads into registers (a chunk's 98 KB of weights, 65 KB
-// of inputs and their halos, at 64 bytes a cycle from the CU's L1; half the
-// weights took 8% off) and, with one workgroup on a CU, the 5 us before its
-// first MFMA and 3 us after its last, of 25.  Alone, l2l + l2g / g2l, f32 MFMAs
-// -> split, us: 2048x2048 332 / 274 -> 217 / 192, 1024x1024 86 / 70 -> 51 / 42.
-// The staging's instructions between the MFMAs instead of behind them: 1%.
+// What bounds it: the loads into registers (a chunk's 147 KB of weights, 65 KB
+// of inputs and their halos, 3300 cycles at 64 bytes a cycle from the CU's L1;
+// its MFMAs take 2304) and, with one workgroup on a CU, what comes before its
+// first MFMA and after its last.  Alone, 128 -> 512 channels, f32 MFMAs / here,
+// us: 256x256 378 / 312, 128x128 98 / 78.  The small products share the sums of
+// the large ones: second sums have no registers.
 #include <hip/hip_runtime.h>
 
 #include "common.h"
@@ -47,8 +47,8 @@ struct W42Cfg {
     static constexpr int KC = 16;          // input channels per chunk
     static constexpr int NU = 6, NTR = 16;  // x positions; tiles per row pair
     static constexpr int NT = 512;
-    static constexpr int RING = 3;  // positions whose weights are in registers (6 spill)
-    static constexpr int VGS = 24 * 32, VPS = 2 * VGS, VBS = 2 * VPS;  // group, part and buffer strides, h8
+    static constexpr int RING = 2;  // positions whose weights are in registers (3 spill: 447 us against 388 in a 2048x2048 pass)
+    static constexpr int VGS = 24 * 32, VPS = 2 * VGS, VBS = 3 * VPS;  // group, part and buffer strides, b8
     static constexpr int X_LDS = 8 * 16 * 64;  // epilogue: 16 registers x 64 lanes of four pixels per wave
     static constexpr int LDS = 2 * VBS > X_LDS ? 2 * VBS : X_LDS;  // 16-byte words
     static_assert(NU % RING == 0, "a ring slot holds the same positions in every chunk");
@@ -69,7 +69,7 @@ __device__ __forceinline__ float w42_bt(const float (&e)[6])
 // One 64-channel x 4-row x 64-pixel block of problem P (no second segment,
 // addends or residual: the FFC's launches store raw partial sums).
 template <class C>
-__device__ __forceinline__ void w42_tile(const ConvProblem &P_mem, int b, h8 *vs, float *slot, float *epl)
+__device__ __forceinline__ void w42_tile(const ConvProblem &P_mem, int b, b8 *vs, float *epl)
 {
     const ConvProblem P = P_mem;  // one batch of scalar loads, held across the barriers
     // K slice of a split problem: the blocks of slice ks follow those of ks - 1
@@ -87,13 +87,13 @@ __device__ __forceinline__ void w42_tile(const ConvProblem &P_mem, int b, h8 *vs
     const ConvSeg &sg = P.s0;
     const unsigned cs = (unsigned)sg.cs;
     const LAMA_GLOBAL float *src = gp(sg.src);
-    // weights: [64 rows][8-channel group][wave][u][part][32][8] halves, 12288 floats a group
-    const LAMA_GLOBAL float *wt = gp(sg.wt) + (long)mb * 64 * sg.wrow + wave * (C::NU * 256);
+    // weights: [64 rows][8-channel group][wave][u][part][32][8], 18432 floats a group
+    const LAMA_GLOBAL float *wt = gp(sg.wt) + (long)mb * 64 * sg.wrow + wave * (C::NU * 384);
     int nc = sg.C, ng = sg.nchunk / 2;  // channels; packed groups (the pack counts chunks of 4, in pairs)
     if (P.ksplit > 1) {
         const int c0 = ks * P.kchunks * 4;
         src += (long)c0 * cs;
-        wt += (long)(c0 / 8) * 12288;
+        wt += (long)(c0 / 8) * 18432;
         ng = P.kchunks / 2;
         nc = min(nc - c0, ng * 8);
     }
@@ -172,49 +172,12 @@ __device__ __forceinline__ void w42_tile(const ConvProblem &P_mem, int b, h8 *vs
                     for (int i = 0; i < 6; ++i) e[c][i] = 0.f;
         }
     };
-    // this wave's largest magnitude, for the workgroup
-    auto publish = [&](float *to, bool finite) {
-        float m = 0.f;
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int i = 0; i < 6; ++i) {
-                const float a = fabsf(e[c][i]);
-                // as bits: a NaN counts as more than an infinity
-                m = finite ? fmaxf(m, a < __builtin_inff() ? a : 0.f)
-                           : __uint_as_float(max(__float_as_uint(m), __float_as_uint(a)));
-            }
-        m = wave_max(m);
-        if (lane == 0) to[wave] = m;
-    };
-    auto agreed = [&](const float *from) {
-        unsigned m = 0;
-#pragma unroll
-        for (int w = 0; w < 8; ++w) m = max(m, __float_as_uint(from[w]));
-        return __uint_as_float((unsigned)__builtin_amdgcn_readfirstlane((int)m));
-    };
-    // the chunk's scale, from the magnitudes published before the last barrier
-    bool inf;
-    auto exponent = [&](int k, int ck) {
-        float m = agreed(slot + 8 * (ck & 1));
-        inf = !(m < __builtin_inff());
-        if (inf) {  // the scale is that of the finite values
-            publish(slot + 16, true);
-            __syncthreads();
-            m = agreed(slot + 16);
-        }
-        return split_exp(k, m, 4);
-    };
-    h4 *const dst = reinterpret_cast<h4 *>(vs + wm * C::VGS + vy * (6 * 32) + rp * 16 + it) + qh;
-    float s = 1.f;
-    auto stage = [&](auto u_, auto inf_, int ck) {
+    b4 *const dst = reinterpret_cast<b4 *>(vs + wm * C::VGS + vy * (6 * 32) + rp * 16 + it) + qh;
+    auto stage = [&](auto u_, auto any, int ck) {
         constexpr int U = decltype(u_)::value;
         const float x[4] = {w42_bt<U>(e[0]), w42_bt<U>(e[1]), w42_bt<U>(e[2]), w42_bt<U>(e[3])};
-        h4 hi, lo;
-        split_n<decltype(inf_)::value>(x, s, hi, lo);
-        h4 *p = dst + 2 * ((ck & 1) * C::VBS + U * 32);
-        p[0] = hi;
-        p[2 * C::VPS] = lo;
+        b4 *p = dst + 2 * ((ck & 1) * C::VBS + U * 32);
+        return split3<decltype(any)::value>(x, p[0], p[2 * C::VPS], p[4 * C::VPS]);
     };
     auto each_u = [&](auto f) {
         f(std::integral_constant<int, 0>{});
@@ -226,85 +189,67 @@ __device__ __forceinline__ void w42_tile(const ConvProblem &P_mem, int b, h8 *vs
     };
     load(0);
     // lane (g, j): output channel wm * 32 + j, group 2 ck + g (past the last: the last, against zeros)
-    h8 wh[C::RING], wl[C::RING];
+    b8 w0[C::RING], w1[C::RING], w2[C::RING];
     auto load_w = [&](int u, int ck) {
-        const unsigned o = (unsigned)(min(2 * ck + g, ng - 1) * 49152 + j * 16);
-        const LAMA_GLOBAL float *p = wt + u * 256;
-        wh[u % C::RING] = *at_byte<h8>(p, o);
-        wl[u % C::RING] = *at_byte<h8>(p, o + 512u);
+        const unsigned o = (unsigned)(min(2 * ck + g, ng - 1) * 73728 + j * 16);
+        const LAMA_GLOBAL float *p = wt + u * 384;
+        w0[u % C::RING] = *at_byte<b8>(p, o);
+        w1[u % C::RING] = *at_byte<b8>(p, o + 512u);
+        w2[u % C::RING] = *at_byte<b8>(p, o + 1024u);
     };
 #pragma unroll
     for (int u = 0; u < C::RING; ++u) load_w(u, 0);
     const int ec = min(m0 + (tid & 63), P.M - 1);
     const float ep = tid < 64    ? (P.bias ? gp(P.bias)[ec] : 0.f)
                      : tid < 128 ? (P.scale ? gp(P.scale)[ec] : 1.f)
-                     : tid < 192 ? (P.scale ? gp(P.shift)[ec] : 0.f)
-                                 : gp(sg.wsc)[ec];
-    if (tid < 256) epl[tid] = ep;
+                                 : (P.scale ? gp(P.shift)[ec] : 0.f);
+    if (tid < 192) epl[tid] = ep;
     f32x16 acc[C::NU];
 #pragma unroll
     for (int u = 0; u < C::NU; ++u)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[u][r] = 0.f;
     combine(0);
-    publish(slot, false);
-    __syncthreads();
-    int k = exponent(SPLIT_K_START, 0);
-    s = pow2f(k);
     load(min(1, n - 1));
-    if (inf)
-        each_u([&](auto u) { stage(u, std::true_type{}, 0); });
-    else
-        each_u([&](auto u) { stage(u, std::false_type{}, 0); });
+    {
+        float check = 0.f;
+        each_u([&](auto u) { check += stage(u, std::false_type{}, 0); });
+        if (split3_again(check)) each_u([&](auto u) { stage(u, std::true_type{}, 0); });
+    }
     combine(min(1, n - 1));
-    publish(slot + 8, false);
     for (int ck = 0; ck < n; ++ck) {
         __syncthreads();  // chunk ck is staged, the other buffer's readers are done
-        const bool more = ck + 1 < n;
-        int kn = k;
-        inf = false;
-        if (more) {
-            kn = exponent(k, ck + 1);
-            s = pow2f(kn);
-        }
         load(min(ck + 2, n - 1));  // unconditional: the waits then count exactly
+        float check = 0.f;
         // each position's operand reads are issued before the position before it
-        h8 xh[2], xl[2];
-        const h8 *const rd = vs + (ck & 1) * C::VBS + g * C::VGS + vy * (6 * 32) + j;
+        b8 x[2][3];
+        const b8 *const rd = vs + (ck & 1) * C::VBS + g * C::VGS + vy * (6 * 32) + j;
         auto read = [&](int u) {
-            xh[u & 1] = rd[u * 32];
-            xl[u & 1] = rd[u * 32 + C::VPS];
+#pragma unroll
+            for (int part = 0; part < 3; ++part) x[u & 1][part] = rd[u * 32 + part * C::VPS];
         };
         read(0);
         each_u([&](auto u_) {
             constexpr int u = decltype(u_)::value;
             if (u + 1 < C::NU) read(u + 1);
-            acc[u] = mfma_split(wh[u % C::RING], wl[u % C::RING], xh[u & 1], xl[u & 1], acc[u]);
+            const auto &v = x[u & 1];
+            mfma_split3(w0[u % C::RING], w1[u % C::RING], w2[u % C::RING], v[0], v[1], v[2], acc[u], acc[u]);
             load_w((u + C::RING) % C::NU, ck + (u + C::RING) / C::NU);
             // after the last chunk this stages that one again, unread
-            stage(u_, std::false_type{}, ck + 1);
-            // the three MFMAs depend on each other: the staging's instructions
+            check += stage(u_, std::false_type{}, ck + 1);
+            // the six MFMAs depend on each other: the staging's instructions
             // go into their waits
 #pragma unroll
-            for (int i = 0; i < 3; ++i) {
+            for (int i = 0; i < 6; ++i) {
                 __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x2, 14, 0);
+                __builtin_amdgcn_sched_group_barrier(0x2, 7, 0);
             }
             // keep the load here: the scheduler would otherwise sink it below
             // the chunk's last MFMA
             __builtin_amdgcn_sched_barrier(0);
         });
-        if (inf) each_u([&](auto u) { stage(u, std::true_type{}, ck + 1); });
+        if (split3_again(check)) each_u([&](auto u) { stage(u, std::true_type{}, ck + 1); });
         combine(min(ck + 2, n - 1));
-        publish(slot + 8 * (ck & 1), false);
-        if (kn != k) {
-            const float f = pow2f(max(kn - k, -126));
-#pragma unroll
-            for (int u = 0; u < C::NU; ++u)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[u][r] *= f;
-            k = kn;
-        }
     }
     __syncthreads();  // every wave has left the K loop: the staging buffers are free
     // A_x^T = (1, 1, 1, 1, 1, 0; 0, 1, -1, 2, -2, 0; 0, 1, 1, 4, 4, 0; 0, 1, -1, 8, -8, 1)
@@ -317,7 +262,6 @@ __device__ __forceinline__ void w42_tile(const ConvProblem &P_mem, int b, h8 *vs
             make_float4(acc[0][r] + p1 + p3, q1 + 2.f * q3, p1 + 4.f * p3, q1 + 8.f * q3 + acc[5][r]);
     }
     __syncthreads();
-    const float u = pow2f(-k);  // |k| <= 100
     const int oy = oy0 + 2 * (j >> 4), ox = ox0 + 4 * (j & 15);
     if (oy >= P.OH || ox >= P.OW) return;
     LAMA_GLOBAL float *out = gp(P.out) + (long)ks * P.out_kstride + (long)oy * P.outW + ox;
@@ -329,10 +273,9 @@ __device__ __forceinline__ void w42_tile(const ConvProblem &P_mem, int b, h8 *vs
 #pragma unroll
         for (int v = 0; v < 4; ++v) q[v] = X[((wm * 4 + v) * 16 + r) * 64];
         if (m0 + cl >= P.M) continue;
-        const float sc = epl[192 + cl] * u, bias = epl[cl], mul = epl[64 + cl], add = epl[128 + cl];
+        const float bias = epl[cl], mul = epl[64 + cl], add = epl[128 + cl];
         auto fin = [&](float x) {  // absent operands are neutral (0, 1, 0)
-            x = x * sc + bias;
-            x = x * mul + add;
+            x = (x + bias) * mul + add;
             return P.relu ? fmaxf(x, 0.f) : x;
         };
 #pragma unroll
@@ -362,13 +305,13 @@ extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_pe
 {
     LAMA_CONV_STARTS;
     LAMA_STAMP_BEGIN;
-    __shared__ h8 vs[W42Cfg<true>::LDS];
-    __shared__ float slot[24], epl[256];
+    __shared__ b8 vs[W42Cfg<true>::LDS];
+    __shared__ float epl[192];
     int b = wino_xcd_order(blockIdx.x, gridDim.x);
     const int pi = find_problem(ps, b);
     if (probs[pi].vec_in && (probs[pi].s0.IW & 3) == 0)
-        w42_tile<W42Cfg<true>>(probs[pi], b, vs, slot, epl);
+        w42_tile<W42Cfg<true>>(probs[pi], b, vs, epl);
     else
-        w42_tile<W42Cfg<false>>(probs[pi], b, vs, slot, epl);
+        w42_tile<W42Cfg<false>>(probs[pi], b, vs, epl);
     LAMA_STAMP_END;
 }

@@ -1,5 +1,5 @@
 // FFC 3x3 convolutions (stride 1, reflect pad 1) as a one-dimensional
-// Winograd F(4,3) along x, on split f16 products (split.h).
+// Winograd F(4,3) along x, on three bf16 parts (split.h).
 //
 // Each output quad (x .. x+3) of a row is computed from the six input columns
 // d0..d5 = in[x-1 .. x+4] of each kernel row ky, with the interpolation points
@@ -16,8 +16,7 @@
 //         out0 = m0 + m1 + m2 + m3 + m4      out2 = m1 + m2 + 4 (m3 + m4)
 //         out1 = m1 - m2 + 2 (m3 - m4)       out3 = m1 - m2 + 8 (m3 - m4) + m5
 // 6 multiplications per 4 outputs and kernel row instead of 12; the
-// transformed values are split (|V| <= 10 max |d|, so the scale is that of d
-// with four bits more).
+// transformed values are split.
 //
 // A workgroup computes 64 output channels x RW rows x 4*NTR pixels (32
 // Winograd tiles: RW rows of NTR tiles, NTR = 16, 8 or 4, so 64-, 32- or
@@ -25,24 +24,23 @@
 // positions u = 3*wu .. 3*wu+2 as three 32 x 32 accumulators: GEMM rows are
 // output channels, GEMM columns the block's 32 tiles, K = (ci, ky).  K is
 // walked in chunks of 16 input channels: the chunk's input rows, loaded into
-// registers during the chunk before, are transformed, scaled, split and stored
-// as [part][8-channel group][row][u][tile][8] halves, so that an MFMA operand
-// is one 16-byte read a lane, over consecutive tiles.  Weights are MFMA
-// operands of one wave each, in operand order, and go straight into registers,
-// a whole chunk (nine steps) ahead: they come from HBM once a pass.  In the
+// registers during the chunk before, are transformed, split and stored as
+// [part][8-channel group][row][u][tile][8], so that an MFMA operand is one
+// 16-byte read a lane, over consecutive tiles.  Weights are MFMA operands of one
+// wave each, in operand order, and go straight into registers, three steps (18
+// MFMAs) ahead: nine steps ahead take 72 registers more, which the second sums of
+// the products use better, at the same speed (512x512: 3.76 ms with nine and one
+// sum, 3.70 with three and two).  In the
 // epilogue the two position halves of each channel half swap partial sums of
 // the output transform through LDS, so that each wave finishes two of the four
 // pixels of every tile.
 //
-// What bounds it: the staging's vector instructions and the weights' latency,
-// no longer the MFMAs (864 of about 5000 cycles a chunk with one workgroup on a
-// CU).  Alone at 512x512, l2l + l2g / g2l: 21.7 / 17.4 us (f32 MFMAs: 36.4 /
-// 28.4).  Measured beside it and not kept, in passes with the other streams:
-// weights three steps ahead instead of nine, which lets three workgroups on a
-// CU (3.63 against 3.50 ms at 512x512, 5.15 against 5.03 at 600x600); 128
-// channels a workgroup, each input staged half as often (3.72 and 5.46 ms with
-// two LDS stages and the staging between the MFMAs: the spectral branch waits
-// for room beside the wider workgroups).
+// What bounds it: the bytes into registers (110 KB of weights and 17 KB of inputs
+// a chunk and workgroup, 2000 cycles at the L1's 64 bytes a cycle), the MFMAs
+// (1728) and the staging's vector instructions (about 1100), which two workgroups
+// on a CU overlap only in part: about 5000 cycles a chunk.  Alone, 128 -> 512
+// channels, f32 MFMAs / here, us: 64x64 36.6 / 31.7, 128x128 112 / 80, 256x256
+// 418 / 296.
 #include <hip/hip_runtime.h>
 
 #include "common.h"
@@ -60,17 +58,17 @@ struct W43Cfg {
     static constexpr int NU = 6, KY = 3;         // Winograd positions, kernel rows
     static constexpr int NUW = NU / 2;           // positions per wave
     static constexpr int NS = KY * NUW;          // steps per wave and chunk
-    static constexpr int RING = 9;               // steps whose weights are in registers
+    static constexpr int RING = 3;               // steps whose weights are in registers
     static constexpr int NTR = NTR_;             // tiles per output row
     static constexpr int RW = 32 / NTR;          // output rows per block
     static constexpr int TR = RW, TC = 4 * NTR;  // output rows x pixels per block
     static constexpr int IR = TR + 2;            // input rows per block
     static constexpr int NITEM = 4 * IR * NTR;   // (4 channels, row, tile) input items per chunk, at most one a thread
-    // LDS, in h8: a row's stride puts the 16 lanes of a read phase, runs of
+    // LDS, in b8: a row's stride puts the 16 lanes of a read phase, runs of
     // NTR tiles in 16 / NTR rows, on distinct banks
     static constexpr int VRS = NTR == 16 ? 96 : NTR == 8 ? 56 : 28;
     static constexpr int VGS = IR * VRS, VPS = 2 * VGS;  // group and part strides
-    static constexpr int V_LDS = 2 * VPS;
+    static constexpr int V_LDS = 3 * VPS;
     // epilogue exchange: per channel half, two pixels x 16 registers x 64 lanes from each position half
     static constexpr int X_LDS = 2 * 2 * 2 * 16 * 64 / 4;
     static constexpr int LDS = V_LDS > X_LDS ? V_LDS : X_LDS;
@@ -92,7 +90,7 @@ __device__ __forceinline__ void w43_bt(const float (&d)[6], float (&v)[6])
 // One 64-channel x RW-row x 4*NTR-pixel block of problem P (no second segment,
 // addends or residual: the FFC's launches store raw partial sums).
 template <class C>
-__device__ __forceinline__ void w43_tile(const ConvProblem &P_mem, int b, h8 *vs, float *slot, float *epl)
+__device__ __forceinline__ void w43_tile(const ConvProblem &P_mem, int b, b8 *vs, float *epl)
 {
     const ConvProblem P = P_mem;  // one batch of scalar loads, held across the barriers
     // K slice of a split problem: the blocks of slice ks follow those of ks - 1
@@ -112,13 +110,13 @@ __device__ __forceinline__ void w43_tile(const ConvProblem &P_mem, int b, h8 *vs
     const ConvSeg &sg = P.s0;
     const unsigned cs = (unsigned)sg.cs;
     const LAMA_GLOBAL float *src = gp(sg.src);
-    // weights: [64 rows][8-channel group][wave][step][part][32][8] halves, 9216 floats a group
-    const LAMA_GLOBAL float *wt = gp(sg.wt) + (long)mb * 64 * sg.wrow + wave * (C::NS * 256);
+    // weights: [64 rows][8-channel group][wave][step][part][32][8], 13824 floats a group
+    const LAMA_GLOBAL float *wt = gp(sg.wt) + (long)mb * 64 * sg.wrow + wave * (C::NS * 384);
     int nc = sg.C, ng = sg.nchunk / 2;  // channels; packed groups (the pack counts chunks of 4, in pairs)
     if (P.ksplit > 1) {
         const int c0 = ks * P.kchunks * 4;
         src += (long)c0 * cs;
-        wt += (long)(c0 / 8) * 9216;
+        wt += (long)(c0 / 8) * 13824;
         ng = P.kchunks / 2;
         nc = min(nc - c0, ng * 8);
     }
@@ -168,44 +166,42 @@ __device__ __forceinline__ void w43_tile(const ConvProblem &P_mem, int b, h8 *vs
     };
     load(0);
     // lane (g, j): output channel wm * 32 + j, group 2 ck + g (past the last: the last, against zeros)
-    h8 wh[C::RING], wl[C::RING];
+    b8 w0[C::RING], w1[C::RING], w2[C::RING];
     auto load_w = [&](int s, int ck) {
-        const unsigned o = (unsigned)(min(2 * ck + g, ng - 1) * 36864 + j * 16);
-        const LAMA_GLOBAL float *p = wt + s * 256;
-        wh[s % C::RING] = *at_byte<h8>(p, o);
-        wl[s % C::RING] = *at_byte<h8>(p, o + 512u);
+        const unsigned o = (unsigned)(min(2 * ck + g, ng - 1) * 55296 + j * 16);
+        const LAMA_GLOBAL float *p = wt + s * 384;
+        w0[s % C::RING] = *at_byte<b8>(p, o);
+        w1[s % C::RING] = *at_byte<b8>(p, o + 512u);
+        w2[s % C::RING] = *at_byte<b8>(p, o + 1024u);
     };
 #pragma unroll
     for (int s = 0; s < C::RING; ++s) load_w(s, 0);
     const int ec = min(m0 + (tid & 63), P.M - 1);
     const float ep = tid < 64    ? (P.bias ? gp(P.bias)[ec] : 0.f)
                      : tid < 128 ? (P.scale ? gp(P.scale)[ec] : 1.f)
-                     : tid < 192 ? (P.scale ? gp(P.shift)[ec] : 0.f)
-                                 : gp(sg.wsc)[ec];
-    f32x16 acc[C::NUW];
+                                 : (P.scale ? gp(P.shift)[ec] : 0.f);
+    f32x16 acc[C::NUW], low[C::NUW];
 #pragma unroll
     for (int q = 0; q < C::NUW; ++q)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[q][r] = 0.f;
-    int k = SPLIT_K_START;
-    // where this item's 4 channels go: V_u at + u * NTR, lo a part on
-    h4 *const dst = reinterpret_cast<h4 *>(vs + (qc >> 1) * C::VGS + ir * C::VRS + it) + (qc & 1);
+        for (int r = 0; r < 16; ++r) acc[q][r] = low[q][r] = 0.f;
+    // where this item's 4 channels go: V_u at + u * NTR, the parts VPS apart
+    b4 *const dst = reinterpret_cast<b4 *>(vs + (qc >> 1) * C::VGS + ir * C::VRS + it) + (qc & 1);
     // the MFMA column's output row and tile within the block
-    const h8 *const rd = vs + g * C::VGS + (j / C::NTR) * C::VRS + j % C::NTR + C::NUW * wu * C::NTR;
-    auto store = [&](auto inf_) {
-        if (C::NITEM < LAMA_NT && tid >= C::NITEM) return;
-        const float s = pow2f(k);
+    const b8 *const rd = vs + g * C::VGS + (j / C::NTR) * C::VRS + j % C::NTR + C::NUW * wu * C::NTR;
+    auto stage = [&](auto any) {
+        float check = 0.f;
+        if (C::NITEM < LAMA_NT && tid >= C::NITEM) return check;
         float v[4][6];
 #pragma unroll
         for (int e = 0; e < 4; ++e) w43_bt(d[e], v[e]);
 #pragma unroll
         for (int u = 0; u < 6; ++u) {
             const float x[4] = {v[0][u], v[1][u], v[2][u], v[3][u]};
-            h4 hi, lo;
-            split_n<decltype(inf_)::value>(x, s, hi, lo);
-            dst[2 * u * C::NTR] = hi;
-            dst[2 * (u * C::NTR + C::VPS)] = lo;
+            b4 *p = dst + 2 * u * C::NTR;
+            check += split3<decltype(any)::value>(x, p[0], p[2 * C::VPS], p[4 * C::VPS]);
         }
+        return check;
     };
     for (int ck = 0; ck < n; ++ck) {
         if ((ck + 1) * C::KC > nc) {
@@ -215,56 +211,23 @@ __device__ __forceinline__ void w43_tile(const ConvProblem &P_mem, int b, h8 *vs
 #pragma unroll
                     for (int i = 0; i < 6; ++i) d[e][i] = 0.f;
         }
-        auto agree = [&](bool finite) {  // the workgroup's largest magnitude
-            float m = 0.f;
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int i = 0; i < 6; ++i) {
-                    const float a = fabsf(d[e][i]);
-                    m = fmaxf(m, finite && !(a < __builtin_inff()) ? 0.f : a);
-                }
-            m = wave_max(m);
-            if (lane == 0) slot[wave] = m;
-            __syncthreads();  // and every wave is done with the last chunk's operands
-            m = fmaxf(fmaxf(slot[0], slot[1]), fmaxf(slot[2], slot[3]));
-            return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(m)));
-        };
-        float m = agree(false);
-        const bool inf = !(m < __builtin_inff());
-        if (inf) {  // the scale is that of the finite values
-            __syncthreads();
-            m = agree(true);
-        }
-        const int kn = split_exp(k, m, 4);
-        if (kn != k) {
-            if (ck > 0) {
-                const float f = pow2f(max(kn - k, -126));
-#pragma unroll
-                for (int q = 0; q < C::NUW; ++q)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[q][r] *= f;
-            }
-            k = kn;
-        }
-        if (inf)
-            store(std::true_type{});
-        else
-            store(std::false_type{});
+        if (ck > 0) __syncthreads();  // every wave is done with the last chunk's operands
+        if (split3_again(stage(std::false_type{}))) stage(std::true_type{});
         if (ck + 1 < n) load(ck + 1);
         __syncthreads();
         // each step's operand reads are issued before the step before it
-        h8 xh[2], xl[2];
+        b8 x[2][3];
         auto read = [&](int s) {
-            const h8 *x = rd + (s / C::NUW) * C::VRS + (s % C::NUW) * C::NTR;
-            xh[s & 1] = x[0];
-            xl[s & 1] = x[C::VPS];
+            const b8 *p = rd + (s / C::NUW) * C::VRS + (s % C::NUW) * C::NTR;
+#pragma unroll
+            for (int part = 0; part < 3; ++part) x[s & 1][part] = p[part * C::VPS];
         };
         read(0);
 #pragma unroll
         for (int s = 0; s < C::NS; ++s) {
             if (s + 1 < C::NS) read(s + 1);
-            acc[s % C::NUW] = mfma_split(wh[s % C::RING], wl[s % C::RING], xh[s & 1], xl[s & 1], acc[s % C::NUW]);
+            const auto &v = x[s & 1];
+            mfma_split3(w0[s % C::RING], w1[s % C::RING], w2[s % C::RING], v[0], v[1], v[2], acc[s % C::NUW], low[s % C::NUW]);
             if (s + C::RING < C::NS)
                 load_w(s + C::RING, ck);
             else
@@ -274,6 +237,8 @@ __device__ __forceinline__ void w43_tile(const ConvProblem &P_mem, int b, h8 *vs
             __builtin_amdgcn_sched_barrier(0);
         }
     }
+#pragma unroll
+    for (int q = 0; q < C::NUW; ++q) acc[q] += low[q];
     // output transform: wave wu = 0 holds m0..m2, wu = 1 holds m3..m5.
     // Partials  p = (m0 + m1 + m2, m1 - m2, m1 + m2, m1 - m2)   (wu = 0)
     //           q = (m3 + m4, 2 (m3 - m4), 4 (m3 + m4), 8 (m3 - m4) + m5)   (wu = 1)
@@ -307,9 +272,8 @@ __device__ __forceinline__ void w43_tile(const ConvProblem &P_mem, int b, h8 *vs
     for (int e = 0; e < 2; ++e)
 #pragma unroll
         for (int r = 0; r < 16; ++r) xl[((wu * 2 + e) * 16 + r) * 64] = give[e][r];
-    epl[tid] = ep;
+    if (tid < 192) epl[tid] = ep;
     __syncthreads();
-    const float u = pow2f(-k);  // |k| <= 100 once a chunk has been taken
     const int oy = oy0 + j / C::NTR, ox = ox0 + 4 * (j % C::NTR) + 2 * wu;
     if (oy >= P.OH || ox >= P.OW) return;
     const bool second = ox + 1 < P.OW;
@@ -324,7 +288,7 @@ __device__ __forceinline__ void w43_tile(const ConvProblem &P_mem, int b, h8 *vs
         float x[2];
 #pragma unroll
         for (int e = 0; e < 2; ++e)
-            x[e] = (mine[e][r] + xl[(((wu ^ 1) * 2 + e) * 16 + r) * 64]) * epl[192 + cl] * u + epl[cl];
+            x[e] = mine[e][r] + xl[(((wu ^ 1) * 2 + e) * 16 + r) * 64] + epl[cl];
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             x[e] = x[e] * epl[64 + cl] + epl[128 + cl];
@@ -371,14 +335,14 @@ __device__ __forceinline__ int wino_xcd_order(int i, int n)
         using C = W43Cfg<NTR, false>;                                                       \
         using C4 = W43Cfg<NTR, true>;                                                       \
         static_assert(C4::LDS == C::LDS, "one LDS layout");                                 \
-        __shared__ h8 vs[C::LDS];                                                           \
-        __shared__ float slot[4], epl[256];                                                 \
+        __shared__ b8 vs[C::LDS];                                                           \
+        __shared__ float epl[192];                                                          \
         int b = wino_xcd_order(blockIdx.x, gridDim.x);                                      \
         const int pi = find_problem(ps, b);                                                 \
         if (probs[pi].vec_in && (probs[pi].s0.IW & 3) == 0)                                 \
-            w43_tile<C4>(probs[pi], b, vs, slot, epl);                                      \
+            w43_tile<C4>(probs[pi], b, vs, epl);                                            \
         else                                                                                \
-            w43_tile<C>(probs[pi], b, vs, slot, epl);                                       \
+            w43_tile<C>(probs[pi], b, vs, epl);                                             \
         LAMA_STAMP_END;                                                                     \
     }
 #ifndef LAMA_W43_WAVES

@@ -281,48 +281,6 @@ void parallel_rows(int n, F f)
     for (std::thread &x : th) x.join();
 }
 
-// f32 to f16 bits, to nearest, ties to even, with subnormals.
-uint16_t f16_bits(float f)
-{
-    uint32_t u;
-    std::memcpy(&u, &f, 4);
-    const uint16_t sign = (uint16_t)(u >> 16 & 0x8000);
-    u &= 0x7fffffff;
-    if (u >= 0x7f800000) return (uint16_t)(sign | (u > 0x7f800000 ? 0x7e00 : 0x7c00));
-    if (u >= 0x477ff000) return (uint16_t)(sign | 0x7c00);  // rounds past the largest half
-    if (u < 0x38800000) {                                    // below 2^-14: a multiple of 2^-24
-        float m;
-        std::memcpy(&m, &u, 4);
-        return (uint16_t)(sign | (uint16_t)std::nearbyint(std::ldexp(m, 24)));
-    }
-    const uint32_t r = u + 0xfff + (u >> 13 & 1);
-    return (uint16_t)(sign | ((r >> 13) - (112 << 10)));
-}
-
-float f16_value(uint16_t h)
-{
-    const int e = h >> 10 & 31, m = h & 1023;
-    const float v = e == 31 ? (m ? NAN : INFINITY) : e ? std::ldexp(1.f + m / 1024.f, e - 15) : std::ldexp((float)m, -24);
-    return h & 0x8000 ? -v : v;
-}
-
-// The scale exponent of a row of weights whose largest finite magnitude is m:
-// m 2^e in [2^14, 2^15), e within +-100 (as the kernels' split_exp).
-int split_row_exp(float m) { return m > 0 ? std::max(-100, std::min(100, 14 - std::ilogb(m))) : 0; }
-
-// hi and lo of v 2^e, as the kernels split activations (split.h).
-void split_f16(float v, int e, uint16_t &hi, uint16_t &lo)
-{
-    if (!std::isfinite(v)) {
-        hi = 0;
-        lo = f16_bits(v);
-        return;
-    }
-    const float x = std::ldexp(v, e);
-    hi = f16_bits(x);
-    lo = f16_bits(x - f16_value(hi));
-}
-
 // v as three bf16 parts, out[0], out[stride] and out[2 stride] (split.h): each
 // the nearest to what the ones before leave, the first towards zero where the
 // nearest would be infinite; infinities and NaNs whole in the third.
@@ -514,17 +472,17 @@ Packed pack_wino(Arena &A, int M, int C, const std::function<float(int, int, int
 // G = (1/4, 0, 0; -1/6, -1/6, -1/6; -1/6, 1/6, -1/6; 1/24, 1/12, 1/6;
 // 1/24, -1/12, 1/6; 0, 0, 1) -- the Winograd F(4,3) weight transform for the
 // points 0, 1, -1, 2, -2, infinity, evaluated in f64 and rounded once to f32
-// -- scaled and split into halves (split_f16) in the order the kernels' waves
-// load them as MFMA operands: per block of 64 output channels (rows past M
-// zero) and group of 8 input channels, [wave (wm, wu)][step s = ky * 3 + q]
-// [hi, lo][32 channels j][8] holds U_u for output channel 32 wm + j and
-// position u = 3 wu + q.  Chunks count 4 channels, in pairs (a group); a block
-// is 64 rows of wrow = nchunk * 72 floats of room.
-// The layout's shape (p.off, p.ws unset).  The same halves are written on the
-// device by lama_pack_wino (kind 4).
+// -- in three bf16 parts (split_bf16) in the order the kernels' waves load them
+// as MFMA operands: per block of 64 output channels (rows past M zero) and
+// group of 8 input channels, [wave (wm, wu)][step s = ky * 3 + q][part][32
+// channels j][8] holds U_u for output channel 32 wm + j and position u = 3 wu
+// + q.  Chunks count 4 channels, in pairs (a group); a block is 64 rows of wrow
+// = nchunk * 108 floats of room.
+// The layout's shape (p.off unset).  The same parts are written on the device
+// by lama_pack_wino (kind 4).
 Packed wino43_shape(int M, int C)
 {
-    constexpr int KC = LAMA_WINO_KC, WK = 72;
+    constexpr int KC = LAMA_WINO_KC, WK = 108;
     static_assert(KC == 4, "a group of 8 is a chunk pair");
     Packed p;
     p.M = M;
@@ -536,7 +494,7 @@ Packed wino43_shape(int M, int C)
     return p;
 }
 
-// floats of a Winograd pack: 64-row blocks (rows past M zero)
+// Floats of a Winograd pack: whole 64-row blocks (wino43_shape, wino42_shape).
 size_t wino_floats(const Packed &p) { return (size_t)((p.M + 63) / 64) * 64 * p.wrow; }
 
 template <class Get>
@@ -546,33 +504,18 @@ Packed pack_wino43(Arena &A, int M, int C, const Get &get)
                                    {1.0 / 24, 1.0 / 12, 1.0 / 6}, {1.0 / 24, -1.0 / 12, 1.0 / 6}, {0, 0, 1}};
     Packed p = wino43_shape(M, C);
     p.off = A.add(wino_floats(p));  // zero: rows past M, channels past C
-    p.ws = A.add(M);
     uint16_t *d = reinterpret_cast<uint16_t *>(A.at(p.off));
-    float *ws = A.at(p.ws);
     parallel_rows(M, [&](int r0, int r1) {
-        std::vector<float> v((size_t)C * 18);
         for (int co = r0; co < r1; ++co) {
-            float most = 0;
+            const int mb = co / 64, wm = co % 64 / 32, j = co % 32;
             for (int ci = 0; ci < C; ++ci) {
                 double g[9];
                 for (int k = 0; k < 9; ++k) g[k] = (double)get(co, ci, k);
+                uint16_t *blk = d + ((size_t)mb * (p.nchunk / 2) + ci / 8) * 27648 + j * 8 + ci % 8;
                 for (int u = 0; u < 6; ++u)
-                    for (int ky = 0; ky < 3; ++ky) {
-                        const float x = (float)(G[u][0] * g[ky * 3] + G[u][1] * g[ky * 3 + 1] + G[u][2] * g[ky * 3 + 2]);
-                        v[(size_t)ci * 18 + u * 3 + ky] = x;
-                        if (std::isfinite(x)) most = std::max(most, std::fabs(x));
-                    }
-            }
-            const int e = split_row_exp(most);
-            ws[co] = std::ldexp(1.f, -e);
-            const int mb = co / 64, wm = co % 64 / 32, j = co % 32;
-            for (int ci = 0; ci < C; ++ci) {
-                uint16_t *blk = d + ((size_t)mb * (p.nchunk / 2) + ci / 8) * 18432 + j * 8 + ci % 8;
-                for (int u = 0; u < 6; ++u)
-                    for (int ky = 0; ky < 3; ++ky) {
-                        uint16_t *at = blk + ((wm * 2 + u / 3) * 9 + ky * 3 + u % 3) * 512;
-                        split_f16(v[(size_t)ci * 18 + u * 3 + ky], e, at[0], at[256]);
-                    }
+                    for (int ky = 0; ky < 3; ++ky)
+                        split_bf16((float)(G[u][0] * g[ky * 3] + G[u][1] * g[ky * 3 + 1] + G[u][2] * g[ky * 3 + 2]),
+                                   blk + ((wm * 2 + u / 3) * 9 + ky * 3 + u % 3) * 768, 256);
             }
         }
     });
@@ -582,18 +525,18 @@ Packed pack_wino43(Arena &A, int M, int C, const Get &get)
 // 3x3 weights for lama_conv3x3w42 (Winograd F(2x4, 3x3)): U(vy, u) =
 // sum over (ky, kx) of Gy[vy][ky] Gx[u][kx] w[ky][kx], Gx the F(4,3) transform
 // of pack_wino43 and Gy = (1, 0, 0; 1/2, 1/2, 1/2; 1/2, -1/2, 1/2; 0, 0, 1) the
-// F(2,3) one, evaluated in f64 and rounded once to f32, scaled and split as
+// F(2,3) one, evaluated in f64 and rounded once to f32, in three bf16 parts as
 // there: per block of 64 output channels (rows past M zero) and group of 8
-// input channels, [wave (wm, vy)][u][hi, lo][32 channels j][8] holds U(vy, u)
+// input channels, [wave (wm, vy)][u][part][32 channels j][8] holds U(vy, u)
 // for output channel 32 wm + j.  Chunks count 4 channels, in pairs (a group); a
-// block is 64 rows of wrow = nchunk * 96 floats of room.
-// The layout's shape (p.off, p.ws unset).  The same halves are written on the
-// device by lama_pack_wino (kind 42).
+// block is 64 rows of wrow = nchunk * 144 floats of room.
+// The layout's shape (p.off unset).  The same parts are written on the device
+// by lama_pack_wino (kind 42).
 Packed wino42_shape(int M, int C)
 {
     Packed p = wino43_shape(M, C);
-    p.T = 64 * 96 / p.KC;
-    p.wrow = p.nchunk * 96;
+    p.T = 64 * 144 / p.KC;
+    p.wrow = p.nchunk * 144;
     return p;
 }
 
@@ -605,33 +548,21 @@ Packed pack_wino42(Arena &A, int M, int C, const Get &get)
     static const double Gy[4][3] = {{1, 0, 0}, {0.5, 0.5, 0.5}, {0.5, -0.5, 0.5}, {0, 0, 1}};
     Packed p = wino42_shape(M, C);
     p.off = A.add(wino_floats(p));  // zero: rows past M, channels past C
-    p.ws = A.add(M);
     uint16_t *d = reinterpret_cast<uint16_t *>(A.at(p.off));
-    float *ws = A.at(p.ws);
     parallel_rows(M, [&](int r0, int r1) {
-        std::vector<float> v((size_t)C * 24);
         for (int co = r0; co < r1; ++co) {
-            float most = 0;
+            const int mb = co / 64, wm = co % 64 / 32, j = co % 32;
             for (int ci = 0; ci < C; ++ci) {
                 double g[3][3], t[4][3];
                 for (int k = 0; k < 9; ++k) g[k / 3][k % 3] = (double)get(co, ci, k);
                 for (int vy = 0; vy < 4; ++vy)  // G_y g
                     for (int kx = 0; kx < 3; ++kx)
                         t[vy][kx] = Gy[vy][0] * g[0][kx] + Gy[vy][1] * g[1][kx] + Gy[vy][2] * g[2][kx];
+                uint16_t *blk = d + ((size_t)mb * (p.nchunk / 2) + ci / 8) * 36864 + wm * 18432 + j * 8 + ci % 8;
                 for (int vy = 0; vy < 4; ++vy)
-                    for (int u = 0; u < 6; ++u) {  // (G_y g) G_x^T
-                        const float x = (float)(Gx[u][0] * t[vy][0] + Gx[u][1] * t[vy][1] + Gx[u][2] * t[vy][2]);
-                        v[(size_t)ci * 24 + vy * 6 + u] = x;
-                        if (std::isfinite(x)) most = std::max(most, std::fabs(x));
-                    }
-            }
-            const int e = split_row_exp(most);
-            ws[co] = std::ldexp(1.f, -e);
-            const int mb = co / 64, wm = co % 64 / 32, j = co % 32;
-            for (int ci = 0; ci < C; ++ci) {
-                uint16_t *blk = d + ((size_t)mb * (p.nchunk / 2) + ci / 8) * 24576 + wm * 12288 + j * 8 + ci % 8;
-                for (int i = 0; i < 24; ++i)
-                    split_f16(v[(size_t)ci * 24 + i], e, blk[i * 512], blk[i * 512 + 256]);
+                    for (int u = 0; u < 6; ++u)  // (G_y g) G_x^T
+                        split_bf16((float)(Gx[u][0] * t[vy][0] + Gx[u][1] * t[vy][1] + Gx[u][2] * t[vy][2]),
+                                   blk + (vy * 6 + u) * 768, 256);
             }
         }
     });
@@ -888,8 +819,7 @@ bool Engine::load_weights(const uint8_t *blob, size_t len, const lama_tensor_inf
                        const lama_tensor_info *s1) {
         p = shape;
         p.off = (dev_n + 63) / 64 * 64;
-        p.ws = p.off + wino_floats(p);
-        dev_n = p.ws + p.M;
+        dev_n = p.off + wino_floats(p);
         dev.push_back({&p, s0, s1, kind});
     };
     const bool dev_wino = dev_pack_ && (wino_ == 4 || wino_ == 42);
@@ -976,10 +906,7 @@ bool Engine::load_weights(const uint8_t *blob, size_t len, const lama_tensor_inf
     // arena: the engine's state changes only once it has succeeded, so a
     // failed load leaves the previous weights and their plans usable
     const size_t dev_base = (A.size() + 63) / 64 * 64, total = dev.empty() ? A.size() : dev_base + dev_n;
-    for (DevJob &j : dev) {
-        j.p->off += dev_base;
-        j.p->ws += dev_base;
-    }
+    for (DevJob &j : dev) j.p->off += dev_base;
     // The device-packed part: zeroed (rows past M, channels past C), the raw
     // matrices copied once each into a temporary buffer, one lama_pack_wino
     // launch over all jobs, then the temporaries freed.
@@ -1017,7 +944,6 @@ bool Engine::load_weights(const uint8_t *blob, size_t len, const lama_tensor_inf
             J.src0 = raw + raw_off[d.s0];
             J.src1 = d.s1 ? raw + raw_off[d.s1] : nullptr;
             J.dst = w + d.p->off;
-            J.wsc = w + d.p->ws;
             J.M = d.p->M;
             J.C = d.p->C;
             J.C0 = (int)d.s0->shape[1];  // input channels from src0; the rest from src1
@@ -1575,7 +1501,6 @@ bool Engine::build_plan(Plan &p, void *arena, std::string &err)
         ConvSeg s{};
         s.src = src;
         s.wt = wp(pk.off);
-        s.wsc = wp(pk.ws);
         s.C = C;
         s.IH = IH;
         s.IW = IW;
@@ -2605,7 +2530,6 @@ SpecPlan *Engine::spec_plan_for(int h, int w, std::string &err)
         ConvProblem q{};
         q.s0.src = src;
         q.s0.wt = wp(pk.off);
-        q.s0.wsc = wp(pk.ws);
         q.s0.C = C;
         q.s0.IH = 1;
         q.s0.IW = N;
@@ -2962,7 +2886,6 @@ bool Engine::op_conv2d(const float *x, int cin, int h, int w, const float *wt, c
     ConvProblem q{};
     q.s0.src = dx;
     q.s0.wt = dw + pk.off;
-    q.s0.wsc = dw + pk.ws;
     q.s0.C = cin;
     q.s0.IH = family == F_CONV1 ? 1 : h;
     q.s0.IW = family == F_CONV1 ? h * w : w;
@@ -3030,7 +2953,6 @@ bool Engine::op_convt(const float *x, int cin, int h, int w, const float *wt, co
         std::memset(&c, 0, sizeof c);
         c.s0.src = dx;
         c.s0.wt = dw + ph[k].off;
-        c.s0.wsc = dw + ph[k].ws;
         c.s0.C = cin;
         c.s0.IH = h;
         c.s0.IW = w;

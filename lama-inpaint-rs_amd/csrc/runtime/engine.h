@@ -27,7 +27,6 @@ size_t step_numel(int step, int h, int w);
 // Convolution weights packed for the MFMA kernels: [M][nchunk][taps][KC].
 struct Packed {
     size_t off = 0;  // float offset in the weight arena
-    size_t ws = 0;   // split packs: offset of the M row scales (ConvSeg::wsc)
     int M = 0, C = 0, T = 0, KC = 0, nchunk = 0, wrow = 0;
 };
 
