@@ -275,12 +275,12 @@ struct TailArgs {
     uint8_t *out_u8;      // lama_tail_u8: composite, HWC [h][w][3]
 };
 
-// One FFC 3x3 weight matrix W[M][C][3][3] to pack into a Winograd kernel's
+// One FFC weight matrix W[M][C][3][3] or W[M][C] to pack into its kernel's
 // layout on the device (lama_pack_wino): input channels ci < C0 come from
 // src0 [M][C0][9], the rest from src1 [M][C - C0][9] (the FFC's local GEMM
 // concatenates l2l and g2l along K).  kind 4: the F(4,3) layout of
-// lama_conv3x3w4*; kind 42: the F(2x4, 3x3) layout of lama_conv3x3w42.
-// Both hold three bf16 parts of every value (split.h).  dst is pre-zeroed (rows
+// lama_conv3x3w4*; kind 42: the F(2x4, 3x3) layout of lama_conv3x3w42; kind 1:
+// W[M][C] for lama_conv1x1* (C0 == C).  All hold three bf16 parts of every value (split.h).  dst is pre-zeroed (rows
 // past M, channels past C stay zero).
 struct WinoPackJob {
     const float *src0, *src1;

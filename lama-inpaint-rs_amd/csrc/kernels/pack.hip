@@ -1,8 +1,8 @@
-// Winograd weight transforms of the FFC 3x3 convolutions, run once when the
-// weights are loaded: each workgroup takes one output channel of one matrix,
-// each of its threads an input channel at a time, reads its nine taps and
-// writes their transformed values into the layout the Winograd kernels load
-// as MFMA operands.
+// The FFCs' weights, packed once when they are loaded: the Winograd transforms of
+// the 3x3 convolutions and the pointwise ones as they are.  Each workgroup takes
+// one output channel of one matrix, each of its threads an input channel at a
+// time, reads its nine taps (its one) and writes their transformed values, in
+// three bf16 parts (split.h), into the layout the kernels load as MFMA operands.
 //
 // The transforms are evaluated in f64 and rounded once to f32, with the same
 // terms summed in the same order as the host packer in engine.cpp
@@ -93,6 +93,14 @@ __device__ __forceinline__ void pack_one_w42(const WinoPackJob &J, int co, int c
 
 }  // namespace
 
+// [32 rows][8-channel group][part][32][8]
+__device__ __forceinline__ void pack_one_pw(const WinoPackJob &J, int co, int ci, float v)
+{
+    put_parts(reinterpret_cast<LAMA_GLOBAL __bf16 *>(gp(J.dst)) + ((long)(co / 32) * 2 * J.nchunk + ci / 8) * 768 +
+                  co % 32 * 8 + ci % 8,
+              v);
+}
+
 // Grid (x: output channels, y: jobs), 256 threads: a workgroup packs one
 // output channel's row; rows past the job's M have nothing to do.
 extern "C" __global__ void __launch_bounds__(256) lama_pack_wino(const WinoPackJob *__restrict__ jobs)
@@ -100,6 +108,10 @@ extern "C" __global__ void __launch_bounds__(256) lama_pack_wino(const WinoPackJ
     const WinoPackJob J = jobs[blockIdx.y];
     const int co = blockIdx.x;
     if (co >= J.M) return;  // whole workgroup
+    if (J.kind == 1) {
+        for (int ci = threadIdx.x; ci < J.C; ci += 256) pack_one_pw(J, co, ci, gp(J.src0)[(long)co * J.C + ci]);
+        return;
+    }
     for (int ci = threadIdx.x; ci < J.C; ci += 256) {
         double g[9];
         const LAMA_GLOBAL float *s = ci < J.C0 ? gp(J.src0) + ((long)co * J.C0 + ci) * 9

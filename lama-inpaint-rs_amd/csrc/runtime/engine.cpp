@@ -386,8 +386,10 @@ Packed pack_tail(Arena &A, int C, const float *w)
 // Pointwise weights [M][C] for the kernels in three bf16 parts: [32 rows][group
 // of 8 channels][part][32][8], rows past M and channels past C zero, the groups
 // rounded up to whole 16-channel steps.
-template <class Get>
-Packed pack_pw(Arena &A, int M, int C, const Get &get)
+// The layout's shape (p.off unset).  The same parts are written on the device by
+// lama_pack_wino (kind 1): the 10.6 M pointwise weights of the network, split
+// here on one thread, were half of the host packing.
+Packed pw_shape(int M, int C)
 {
     Packed p;
     p.M = M;
@@ -396,12 +398,23 @@ Packed pack_pw(Arena &A, int M, int C, const Get &get)
     p.KC = 16;
     p.nchunk = (C + 15) / 16;
     p.wrow = p.nchunk * 24;
-    p.off = A.add((size_t)((M + 31) / 32) * 32 * p.wrow);
+    return p;
+}
+
+size_t pw_floats(const Packed &p) { return (size_t)((p.M + 31) / 32) * 32 * p.wrow; }
+
+template <class Get>
+Packed pack_pw(Arena &A, int M, int C, const Get &get)
+{
+    Packed p = pw_shape(M, C);
+    p.off = A.add(pw_floats(p));
     uint16_t *d = reinterpret_cast<uint16_t *>(A.at(p.off));
-    for (int co = 0; co < M; ++co) {
-        uint16_t *blk = d + (size_t)(co / 32) * 64 * p.wrow + (co % 32) * 8;
-        for (int ci = 0; ci < C; ++ci) split_bf16(get(co, ci), blk + (size_t)(ci / 8) * 768 + ci % 8, 256);
-    }
+    parallel_rows(M, [&](int r0, int r1) {
+        for (int co = r0; co < r1; ++co) {
+            uint16_t *blk = d + (size_t)(co / 32) * 64 * p.wrow + (co % 32) * 8;
+            for (int ci = 0; ci < C; ++ci) split_bf16(get(co, ci), blk + (size_t)(ci / 8) * 768 + ci % 8, 256);
+        }
+    });
     return p;
 }
 
@@ -804,10 +817,11 @@ bool Engine::load_weights(const uint8_t *blob, size_t len, const lama_tensor_inf
         return co < 128 ? w[((size_t)co * 256 + ci) * 9 + t] : w2[((size_t)(co - 128) * 256 + ci) * 9 + t];
     });
     if (!fold_bns(A, S, {{"model.4.bn_l", 128}, {"model.4.bn_g", 384}}, down_bn_[2], err)) return false;
-    // The Winograd packs of the FFC 3x3 convolutions (F(4,3), and F(2x4, 3x3)
-    // for the large planes: 692 of the 749 MB of packed weights) are made on
-    // the device from the raw weights (149 MB), laid out after the host-packed
-    // part of the arena (offsets relative to that part's end until the upload).
+    // The FFCs' weights (the Winograd packs of the 3x3 convolutions, F(4,3) and
+    // F(2x4, 3x3) for the large planes, 1040 MB, and the pointwise ones, 64 of
+    // the 1123 MB of packed weights) are made on the device from the raw
+    // weights (191 MB), laid out after the host-packed part of the arena
+    // (offsets relative to that part's end until the upload).
     struct DevJob {
         Packed *p;
         const lama_tensor_info *s0, *s1;
@@ -819,7 +833,7 @@ bool Engine::load_weights(const uint8_t *blob, size_t len, const lama_tensor_inf
                        const lama_tensor_info *s1) {
         p = shape;
         p.off = (dev_n + 63) / 64 * 64;
-        dev_n = p.off + wino_floats(p);
+        dev_n = p.off + (kind == 1 ? pw_floats(p) : wino_floats(p));
         dev.push_back({&p, s0, s1, kind});
     };
     const bool dev_wino = dev_pack_ && (wino_ == 4 || wino_ == 42);
@@ -835,10 +849,14 @@ bool Engine::load_weights(const uint8_t *blob, size_t len, const lama_tensor_inf
             const lama_tensor_info *tl2g = tg2l ? S.find(pf + ".convl2g.weight", {384, 128, 3, 3}, err) : nullptr;
             if (!tl2g || (!dev_wino && (!S.get(pf + ".convl2l.weight", {128, 128, 3, 3}, l2l, err) ||
                                         !S.get(pf + ".convg2l.weight", {128, 384, 3, 3}, g2l, err) ||
-                                        !S.get(pf + ".convl2g.weight", {384, 128, 3, 3}, l2g, err))) ||
-                !S.get(pf + ".convg2g.conv1.0.weight", {192, 384, 1, 1}, c1, err) ||
-                !S.get(pf + ".convg2g.fu.conv_layer.weight", {384, 384, 1, 1}, fu, err) ||
-                !S.get(pf + ".convg2g.conv2.weight", {384, 192, 1, 1}, c2, err))
+                                        !S.get(pf + ".convl2g.weight", {384, 128, 3, 3}, l2g, err))))
+                return false;
+            const lama_tensor_info *tc1 = S.find(pf + ".convg2g.conv1.0.weight", {192, 384, 1, 1}, err);
+            const lama_tensor_info *tfu = tc1 ? S.find(pf + ".convg2g.fu.conv_layer.weight", {384, 384, 1, 1}, err) : nullptr;
+            const lama_tensor_info *tc2 = tfu ? S.find(pf + ".convg2g.conv2.weight", {384, 192, 1, 1}, err) : nullptr;
+            if (!tc2 || (!dev_pack_ && (!S.get(pf + ".convg2g.conv1.0.weight", {192, 384, 1, 1}, c1, err) ||
+                                        !S.get(pf + ".convg2g.fu.conv_layer.weight", {384, 384, 1, 1}, fu, err) ||
+                                        !S.get(pf + ".convg2g.conv2.weight", {384, 192, 1, 1}, c2, err))))
                 return false;
             if (dev_wino) {
                 // the F(2x4) packs beside the default F(4,3) ones, for the large planes
@@ -867,9 +885,15 @@ bool Engine::load_weights(const uint8_t *blob, size_t len, const lama_tensor_inf
                         : wino_      ? pack_wino(A, 384, 128, l2gw)
                                      : pack(A, 384, 128, 9, 8, l2gw);
             }
-            F.conv2 = pack_pw(A, 384, 192, [&](int co, int ci) { return c2[(size_t)co * 192 + ci]; });
-            F.conv1 = pack_pw(A, 192, 384, [&](int co, int ci) { return c1[(size_t)co * 384 + ci]; });
-            F.fu = pack_pw(A, 384, 384, [&](int co, int ci) { return fu[(size_t)co * 384 + ci]; });
+            if (dev_pack_) {
+                dev_job(F.conv2, pw_shape(384, 192), 1, tc2, nullptr);
+                dev_job(F.conv1, pw_shape(192, 384), 1, tc1, nullptr);
+                dev_job(F.fu, pw_shape(384, 384), 1, tfu, nullptr);
+            } else {
+                F.conv2 = pack_pw(A, 384, 192, [&](int co, int ci) { return c2[(size_t)co * 192 + ci]; });
+                F.conv1 = pack_pw(A, 192, 384, [&](int co, int ci) { return c1[(size_t)co * 384 + ci]; });
+                F.fu = pack_pw(A, 384, 384, [&](int co, int ci) { return fu[(size_t)co * 384 + ci]; });
+            }
             if (!fold_bns(A, S, {{pf + ".convg2g.conv1.1", 192}}, F.bn1, err) ||
                 !fold_bns(A, S, {{pf + ".convg2g.fu.bn", 384}}, F.fu_bn, err) ||
                 !fold_bns(A, S, {{pb + ".bn_l", 128}}, F.bn_l, err) || !fold_bns(A, S, {{pb + ".bn_g", 384}}, F.bn_g, err))
@@ -1002,7 +1026,7 @@ bool Engine::load_weights(const uint8_t *blob, size_t len, const lama_tensor_inf
     if (flag_profile_)
         fprintf(stderr,
                 "gpu weights: %.3fs, %.1f MB resident (host packing %.3fs, arena allocation and upload of %.1f MB %.3fs, "
-                "raw 3x3 upload and Winograd packing on the device %.3fs)\n",
+                "raw upload and packing on the device %.3fs)\n",
                 since(t_load), total * 4 / 1e6, t_host, A.size() * 4 / 1e6, t_upload, t_device);
     have_weights_ = true;
     return true;

@@ -127,6 +127,12 @@ def run_plan_failure():
     eng.close()
 
 
-{"plans": run_plans, "reload_failure": run_reload_failure, "plan_failure": run_plan_failure}[name]()
+def run_load():
+    eng = E.Engine()
+    eng.load_weights(H.Store(weights))  # LAMA_PROFILE=1: its phases on stderr
+    eng.close()
+
+
+{"load": run_load, "plans": run_plans, "reload_failure": run_reload_failure, "plan_failure": run_plan_failure}[name]()
 out["violations"] = fake.fakehip_violations()
 print(json.dumps(out))

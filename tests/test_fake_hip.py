@@ -9,6 +9,7 @@ memory), a failed plan allocation is an error the context recovers from, and
 the no-allocation entry point allocates nothing."""
 import json
 import os
+import re
 import subprocess
 import sys
 
@@ -32,13 +33,17 @@ def weights_file(pkg, tmp_path_factory):
     return p
 
 
-def _scenario(name, fake_lib, weights_file):
-    env = dict(os.environ)
+def _run(name, fake_lib, weights_file, **more):
+    env = dict(os.environ, **more)
     env.pop("FAKEHIP_FAIL_MALLOC_ABOVE", None)
     r = subprocess.run([sys.executable, os.path.join(HERE, "fakehip", "scenarios.py"), name, fake_lib, weights_file],
                        capture_output=True, text=True, env=env, timeout=600)
     assert r.returncode == 0, r.stderr[-3000:]
-    return json.loads(r.stdout.strip().splitlines()[-1])
+    return r
+
+
+def _scenario(name, fake_lib, weights_file):
+    return json.loads(_run(name, fake_lib, weights_file).stdout.strip().splitlines()[-1])
 
 
 def test_every_shape_plans_and_issues_its_launches(fake_lib, weights_file):
@@ -115,3 +120,15 @@ def test_failed_plan_allocation_is_an_error_and_noalloc_allocates_nothing(fake_l
     assert "captured" in o["noalloc_capture"], o["noalloc_capture"]
     assert "600" in o["noalloc_600"] or "scratch" in o["noalloc_600"], o["noalloc_600"]
     assert o["violations"] == 0
+
+
+def test_the_ffc_weights_are_packed_on_the_device(fake_lib, weights_file):
+    """Splitting the FFCs' 48 M weights on the host costs a command line run more
+    than its passes: the host packs and uploads only the other layers' (3.1 M
+    weights, 19 MB as three bf16 parts, and the folded batch norms)."""
+    err = _run("load", fake_lib, weights_file, LAMA_PROFILE="1").stderr
+    mb = re.search(r"arena allocation and upload of ([0-9.]+) MB", err)
+    assert mb and 5 < float(mb.group(1)) < 30, err
+    err = _run("load", fake_lib, weights_file, LAMA_PROFILE="1", LAMA_HOST_PACK="1").stderr
+    mb = re.search(r"arena allocation and upload of ([0-9.]+) MB", err)
+    assert mb and float(mb.group(1)) > 1000, err
