@@ -1191,12 +1191,15 @@ int Engine::ksplit_for(int h, int w) const
 
 // The FFC 3x3 algorithm of an h8 x w8 bottleneck plane: LAMA_FFC_WINO's,
 // except that the default F(4,3) hands the plane to F(2x4, 3x3) where the
-// l2l + l2g launch has at least two of its workgroups (64 channels x 4 rows
-// x 64 pixels) per CU, its 64-pixel columns overhang the plane by at most an
-// eighth of its width, and its rounds of one workgroup per CU are at least
-// 8/9 full: square inputs of 1024 and up.  Measured (ms a pass, F(4,3) /
-// F(2x4)): 2048x2048 29.5 / 28.9, 1024x1024 7.8 / 8.0, 512x512 2.65 / 3.40 (128
-// workgroups), 1088x1920 16.6 / 17.5 (1088 workgroups, 4.25 rounds).
+// l2l + l2g launch has at least four rounds of its workgroups (64 channels x 4
+// rows x 64 pixels, one per CU), its 64-pixel columns overhang the plane by at
+// most an eighth of its width, and the rounds are at least 8/9 full: square
+// inputs of 1472 and up.  Measured, each in a process of its own (ms a pass,
+// F(4,3) / F(2x4), rounds): 1024x1024 9.98 / 10.36 (2), 1024x1536 15.74 / 16.04
+// (3), 1024x2048 20.42 / 20.49 (4), 1536x1536 23.12 / 23.12 (4.5), 1280x2048
+// 25.58 / 25.52 (5), 1536x2048 30.97 / 30.92 (6), 2048x1984 42.81 / 42.70 (8),
+// 2048x2048 38.51 / 38.22 (8); rounds not full: 1152x1536 17.79 / 18.18 (3.4),
+// 1088x1920 21.11 / 21.67 (4.25); overhang 1/5: 1280x1280 16.34 / 17.51.
 // LAMA_W42=0 (read at open) keeps F(4,3) everywhere.
 int Engine::wino_for(int h8, int w8) const
 {
@@ -1204,7 +1207,7 @@ int Engine::wino_for(int h8, int w8) const
     const long blocks = (long)((h8 + 3) / 4) * ((w8 + 63) / 64) * (512 / 64);
     const int overhang = (w8 + 63) / 64 * 64 - w8;
     const long slots = (blocks + LAMA_CUS - 1) / LAMA_CUS * LAMA_CUS;
-    return blocks >= 2 * LAMA_CUS && 8 * overhang <= w8 && 8 * slots <= 9 * blocks ? 42 : 4;
+    return blocks >= 4 * LAMA_CUS && 8 * overhang <= w8 && 8 * slots <= 9 * blocks ? 42 : 4;
 }
 
 // Groups of 4 elements per finalize thread (1 or 2): two where one group per

@@ -425,13 +425,13 @@ def test_device_packed_weights_match_host_packed(pkg, weights_dir, engine):
     """The FFC 3x3 weights packed for the Winograd kernels on the device
     (lama_pack_wino, the default) and on the host (LAMA_HOST_PACK=1): the same
     floats, so forwards through the F(4,3) packs (128 x 96) and through the
-    F(2x4, 3x3) packs (1024 x 1024) are bit-identical."""
+    F(2x4, 3x3) packs (1024 x 2048) are bit-identical."""
     with pytest.MonkeyPatch.context() as mp:
         mp.setenv("LAMA_HOST_PACK", "1")
         eh = pkg.hip_engine.Engine()
     try:
         eh.load_weights(pkg.host_api.Store(weights_dir["cal"]))
-        for (h, w), f2x4 in (((128, 96), False), ((1024, 1024), True)):
+        for (h, w), f2x4 in (((128, 96), False), ((1024, 2048), True)):
             img, mask = _case(pkg, h, w, "strokes")
             x = pkg.host_api.build_input(img, mask)
             print(f"case device vs host packs {h}x{w}", flush=True)
@@ -499,13 +499,14 @@ def test_forward_ksplit_variants_256(pkg, engine, oracle_cal, monkeypatch, ks):
                                             (600, 592, "lama_conv3x3w4q", "lama_rfft2"),
                                             (256, 256, "lama_conv3x3w4n", "lama_rfft2_32"),
                                             (16, 1024, "lama_conv3x3w4", "lama_rfft2"),
-                                            (1024, 1024, "lama_conv3x3w42", "lama_rfft2_rows_128")])
+                                            (1024, 1024, "lama_conv3x3w4", "lama_rfft2_rows_128"),
+                                            (1024, 2048, "lama_conv3x3w42", "lama_rfft2_rows")])
 def test_ffc_block_shape_per_plane(pkg, engine, h, w, kernel, fft):
     """The FFC GEMMs take the F(4,3) block shape that covers the bottleneck
     plane with the fewest blocks of 32 tiles (2 x 64 px on a tie): 75-rows
     planes 10 x 5 blocks of 8 x 16 instead of 19 x 3 of 4 x 32; a plane of 2
     rows and 128 columns 2 blocks of 2 x 64 instead of 4 of 4 x 32.  From
-    128 x 128 bottleneck planes (1024 x 1024 inputs) on they run as F(2x4,
+    four rounds of its blocks on (1024 x 2048 inputs) they run as F(2x4,
     3x3).  Square 32, 64 and 75 planes take the FFT kernels with the shape
     compiled in."""
     print(f"case block shape {h}x{w}", flush=True)
