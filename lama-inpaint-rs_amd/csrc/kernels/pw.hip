@@ -221,8 +221,8 @@ __device__ __forceinline__ void pw_tile(const ConvProblem &P_mem, int b, b8 *xs,
                 acc[h][q] = (kh ? acc[h][8 + q] : acc[h][q]) + ex[(h * 16 + (kh ^ 1) * 8 + q) * 64];
     }
     constexpr int NQ = C::KH ? 8 : 16;
-    // Register q: channel m0 + 32 wm + 8 (q / 4) + q % 4 + 4 g.  FULL: all 32
-    // channels exist, and an address is a uniform row base and a lane offset.
+    // Register q: channel row0 + 8 (q / 4) + q % 4 + 4 g.  FULL: all of the wave's
+    // 2 NQ channels exist, and an address is a uniform row base and a lane offset.
     const int row0 = m0 + 32 * wm + (C::KH ? 16 * kh : 0);
     auto finish = [&](auto full_) {
         constexpr bool FULL = decltype(full_)::value;
@@ -265,7 +265,7 @@ __device__ __forceinline__ void pw_tile(const ConvProblem &P_mem, int b, b8 *xs,
             }
         }
     };
-    if (row0 + 32 <= P.M)
+    if (row0 + 2 * NQ <= P.M)
         finish(std::true_type{});
     else
         finish(std::false_type{});

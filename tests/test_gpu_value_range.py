@@ -17,10 +17,12 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-5
 
 # kind: (cin, cout, h, w) of one tile or a few.  pw: the 32-pixel and the
-# 64-pixel tiles; w43, w42: F(4,3) and F(2x4, 3x3)
-CASES = [("pw", 24, 96, 5, 9), ("pw", 13, 33, 6, 7), ("pw", 96, 65, 190, 188), ("w43", 24, 70, 6, 36),
-         ("w43", 13, 8, 11, 75), ("w42", 24, 70, 8, 36), ("w42", 13, 8, 11, 75), ("down", 24, 70, 19, 24),
-         ("up", 24, 70, 9, 24), ("head", 4, 64, 19, 33), ("head", 3, 33, 9, 40), ("tail", 40, 3, 17, 60)]
+# 64-pixel tiles, with 48 and 80 channels ending in the middle of the 32 that two
+# waves share; w43, w42: F(4,3) and F(2x4, 3x3)
+CASES = [("pw", 24, 96, 5, 9), ("pw", 13, 33, 6, 7), ("pw", 24, 48, 5, 9), ("pw", 96, 65, 190, 188),
+         ("pw", 40, 80, 190, 188), ("w43", 24, 70, 6, 36), ("w43", 13, 8, 11, 75), ("w42", 24, 70, 8, 36),
+         ("w42", 13, 8, 11, 75), ("down", 24, 70, 19, 24), ("up", 24, 70, 9, 24), ("head", 4, 64, 19, 33),
+         ("head", 3, 33, 9, 40), ("tail", 40, 3, 17, 60)]
 
 
 @pytest.fixture(scope="module")
