@@ -517,7 +517,7 @@ extern "C" __global__ void __launch_bounds__(LAMA_FFT_NT) lama_irfft2(const FftA
     } else {
         for (int idx = threadIdx.x; idx < H * W; idx += blockDim.x) {
             int x;
-        const int y = dw.div(idx, x);
+            const int y = dw.div(idx, x);
             const float2 v = q[(y >> 1) * W + x];
             d[idx] = ((y & 1) ? v.y : v.x) * A.scale + ks_ld(f, idx, kf);
         }

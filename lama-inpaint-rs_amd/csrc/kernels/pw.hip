@@ -39,21 +39,20 @@
 
 namespace {
 
-template <int NPX_, int MW_, bool KH_, int KC_>
+template <int NPX_, int MW_, int KC_>
 struct PwCfg {
     static constexpr int NPX = NPX_, MW = MW_, KC = KC_;  // pixels; waves along M; channels per fill
-    static constexpr bool KH = KH_;
-    static constexpr int WAVES = MW * (KH ? 2 : 1), NT = 64 * WAVES;
+    static constexpr int WAVES = 2 * MW, NT = 64 * WAVES;
     static constexpr int MB = 32 * MW, NCB = NPX / 32;
     static constexpr int KG = KC / 8, KS = KC / 16;         // groups and 16-channel steps per fill
-    static constexpr int WS = KH ? KS / 2 : KS;             // steps per wave and fill
+    static constexpr int WS = KS / 2;                       // steps per wave and fill
     static constexpr int RING = WS % 4 == 0 ? 4 : 3;        // weight steps in registers
     static constexpr int PER = KG * NPX / NT, GPR = NT / NPX;  // runs per thread; groups per round of runs
     static constexpr int GPW = 64 / NPX;                    // groups per wave of a round
     static constexpr int XP = KG * NPX, XL = 3 * XP;        // LDS b8s of one part, of the three
     static_assert(PER * NT == KG * NPX && (NPX == 32 || NPX == 64), "whole runs");
     static_assert(WS % RING == 0, "the ring holds a whole number of laps per fill");
-    static_assert(!KH || MW * NCB * 16 * 64 * 4 <= XL * 16, "the halves' exchange fits the strip's LDS");
+    static_assert(MW * NCB * 16 * 64 * 4 <= XL * 16, "the halves' exchange fits the strip's LDS");
 };
 
 // One MB x NPX tile of problem P.
@@ -91,7 +90,7 @@ __device__ __forceinline__ void pw_tile(const ConvProblem &P_mem, int b, b8 *xs,
 #endif
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, j = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = C::KH ? wave >> 1 : wave, kh = C::KH ? wave & 1 : 0;
+    const int wm = wave >> 1, kh = wave & 1;
     const int m0 = mb * C::MB, ox0 = t * C::NPX;
     const ConvSeg &sg = P.s0;
     const int N = sg.IH * sg.IW;
@@ -144,7 +143,7 @@ __device__ __forceinline__ void pw_tile(const ConvProblem &P_mem, int b, b8 *xs,
     b8 w0[C::RING], w1[C::RING], w2[C::RING];
     const unsigned woff = (unsigned)(g * 1536 + j * 16);
     auto load_w = [&](int sl, int f, int s) {
-        const int k16 = min(f * C::KS + (C::KH ? 2 * s + kh : s), n16 - 1);
+        const int k16 = min(f * C::KS + 2 * s + kh, n16 - 1);
         const LAMA_GLOBAL float *p = wt + (long)k16 * 768;
         w0[sl] = *at_byte<b8>(p, woff);
         w1[sl] = *at_byte<b8>(p, woff + 512u);
@@ -185,11 +184,11 @@ __device__ __forceinline__ void pw_tile(const ConvProblem &P_mem, int b, b8 *xs,
         // laps of the ring; the steps of a lap past the last channel multiply zeros
 #pragma unroll
         for (int lap = 0; lap < C::WS; lap += C::RING) {
-            if (f * C::KS + (C::KH ? 2 * lap : lap) >= n16) break;
+            if (f * C::KS + 2 * lap >= n16) break;
 #pragma unroll
             for (int i = 0; i < C::RING; ++i) {
                 const int s = lap + i;
-                const b8 *x = xs + (2 * (C::KH ? 2 * s + kh : s) + g) * C::NPX + j;
+                const b8 *x = xs + (2 * (2 * s + kh) + g) * C::NPX + j;
 #pragma unroll
                 for (int h = 0; h < C::NCB; ++h)
                     mfma_split3(w0[i], w1[i], w2[i], x[32 * h], x[32 * h + C::XP], x[32 * h + 2 * C::XP], acc[h],
@@ -206,24 +205,22 @@ __device__ __forceinline__ void pw_tile(const ConvProblem &P_mem, int b, b8 *xs,
     for (int h = 0; h < C::NCB; ++h) acc[h] += low[h];
     // K halves: each of the two waves finishes eight of the 16 register rows,
     // handing the other eight over
-    if constexpr (C::KH) {
-        float *ex = reinterpret_cast<float *>(xs) + wm * C::NCB * 16 * 64 + lane;
-        __syncthreads();
+    float *ex = reinterpret_cast<float *>(xs) + wm * C::NCB * 16 * 64 + lane;
+    __syncthreads();
 #pragma unroll
-        for (int h = 0; h < C::NCB; ++h)
+    for (int h = 0; h < C::NCB; ++h)
 #pragma unroll
-            for (int q = 0; q < 8; ++q) ex[(h * 16 + kh * 8 + q) * 64] = kh ? acc[h][q] : acc[h][8 + q];
-        __syncthreads();
+        for (int q = 0; q < 8; ++q) ex[(h * 16 + kh * 8 + q) * 64] = kh ? acc[h][q] : acc[h][8 + q];
+    __syncthreads();
 #pragma unroll
-        for (int h = 0; h < C::NCB; ++h)
+    for (int h = 0; h < C::NCB; ++h)
 #pragma unroll
-            for (int q = 0; q < 8; ++q)
-                acc[h][q] = (kh ? acc[h][8 + q] : acc[h][q]) + ex[(h * 16 + (kh ^ 1) * 8 + q) * 64];
-    }
-    constexpr int NQ = C::KH ? 8 : 16;
+        for (int q = 0; q < 8; ++q)
+            acc[h][q] = (kh ? acc[h][8 + q] : acc[h][q]) + ex[(h * 16 + (kh ^ 1) * 8 + q) * 64];
+    constexpr int NQ = 8;
     // Register q: channel row0 + 8 (q / 4) + q % 4 + 4 g.  FULL: all of the wave's
     // 2 NQ channels exist, and an address is a uniform row base and a lane offset.
-    const int row0 = m0 + 32 * wm + (C::KH ? 16 * kh : 0);
+    const int row0 = m0 + 32 * wm + 16 * kh;
     auto finish = [&](auto full_) {
         constexpr bool FULL = decltype(full_)::value;
         const long ocs = P.out_cstride;
@@ -273,14 +270,14 @@ __device__ __forceinline__ void pw_tile(const ConvProblem &P_mem, int b, b8 *xs,
 
 }  // namespace
 
-#define LAMA_PW_KERNEL(NAME, NPX, MW, KH, KC, RES)                                                      \
-    extern "C" __global__ void __launch_bounds__((PwCfg<NPX, MW, KH, KC>::NT))                          \
+#define LAMA_PW_KERNEL(NAME, NPX, MW, KC, RES)                                                          \
+    extern "C" __global__ void __launch_bounds__((PwCfg<NPX, MW, KC>::NT))                              \
         __attribute__((amdgpu_waves_per_eu(NPX == 64 ? 3 : 4))) NAME(LAMA_CONV_PARAMS)                  \
     {                                                                                                   \
         side_priority();                                                                                \
         LAMA_CONV_STARTS;                                                                               \
         LAMA_STAMP_BEGIN;                                                                               \
-        using C = PwCfg<NPX, MW, KH, KC>;                                                               \
+        using C = PwCfg<NPX, MW, KC>;                                                                   \
         __shared__ b8 xs[C::XL];                                                                        \
         __shared__ float epl[3 * C::MB];                                                                \
         int b = blockIdx.x;                                                                             \
@@ -288,8 +285,8 @@ __device__ __forceinline__ void pw_tile(const ConvProblem &P_mem, int b, b8 *xs,
         pw_tile<C, RES>(probs[pi], b, xs, epl);                                                         \
         LAMA_STAMP_END;                                                                                 \
     }
-LAMA_PW_KERNEL(lama_conv1x1, 64, LAMA_PW_MB / 32, true, LAMA_PW_KC, false)
-LAMA_PW_KERNEL(lama_conv1x1_kh, 32, LAMA_PW_KH_MB / 32, true, 192, false)
-LAMA_PW_KERNEL(lama_conv1x1_res, 64, LAMA_PW_MB / 32, true, LAMA_PW_KC, true)
-LAMA_PW_KERNEL(lama_conv1x1_res_kh, 32, LAMA_PW_KH_MB / 32, true, 192, true)
+LAMA_PW_KERNEL(lama_conv1x1, 64, LAMA_PW_MB / 32, LAMA_PW_KC, false)
+LAMA_PW_KERNEL(lama_conv1x1_kh, 32, LAMA_PW_KH_MB / 32, 192, false)
+LAMA_PW_KERNEL(lama_conv1x1_res, 64, LAMA_PW_MB / 32, LAMA_PW_KC, true)
+LAMA_PW_KERNEL(lama_conv1x1_res_kh, 32, LAMA_PW_KH_MB / 32, 192, true)
 #undef LAMA_PW_KERNEL

@@ -1084,7 +1084,6 @@ hipFunction_t Engine::conv_fn(int family, const ConvProblem *probs, size_t n, in
         return fn_edge_q_[family == F_CONVT];
     if ((family == F_CONV1 || family == F_CONV1R) && tile_variant(family, probs[0].OH, probs[0].OW, probs[0].M) == 0)
         return fn_pw_kh_[family == F_CONV1R];
-    (void)n;
     return fn_[family];
 }
 
