@@ -1,11 +1,10 @@
-"""The kernels that multiply f32 values as split f16 halves, where the split can
-go wrong: the common scale of a workgroup (tiny and huge values, values that
-grow along the channels and so lower the scale midway), ragged channel counts
-against the 8- and 16-channel groups, infinities and NaNs.
+"""The kernels that multiply f32 values as three bf16 parts, where the split can
+go wrong: tiny and huge values, values that grow or fall along the channels,
+ragged channel counts against the 8- and 16-channel groups, infinities and NaNs.
 
-Tolerance: a split product is within 2^-22 + 2^-22 of the f32 one and the sum
-of up to 1152 of them is rounded in f32 as before, so the 1e-5 relative bound of
-the other operator tests holds with the same margin, at any scale."""
+Tolerance: a product in parts is within 2^-23 of the f32 one and the sum of up
+to 1152 of them is rounded in f32 as before, so the 1e-5 relative bound of the
+other operator tests holds with the same margin, at any scale."""
 import numpy as np
 import pytest
 

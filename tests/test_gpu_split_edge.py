@@ -1,10 +1,10 @@
-"""The stride-2 and the transposed convolutions as split f16 products, at the
+"""The stride-2 and the transposed convolutions on three bf16 parts, at the
 edges of their tiles (128 pixels, 64 channels), channel chunks (16, by groups
 of 8) and value ranges, against the oracle.
 
-Tolerance: a split product is within 2^-22 + 2^-22 of the f32 one and the sum
-of up to 9 * 100 of them is rounded in f32 as before, so the 1e-5 relative
-bound of the other operator tests holds with the same margin, at any scale."""
+Tolerance: a product in parts is within 2^-23 of the f32 one and the sum of
+up to 9 * 100 of them is rounded in f32 as before, so the 1e-5 relative bound of
+the other operator tests holds with the same margin, at any scale."""
 import numpy as np
 import pytest
 
@@ -48,7 +48,7 @@ def test_any_magnitude(engine, kind, cin, cout, h, w):
     for sx, sw in ((1.0, 1.0), (2.0**-90, 2.0**20), (2.0**60, 2.0**-30)):
         got = _run(engine, kind, x * np.float32(sx), wt * np.float32(sw))
         assert rel_err(got.astype(np.float64) / (sx * sw), ref) < TOL
-    for s in (np.logspace(-6, 6, cin), np.logspace(6, -6, cin)):  # a scale lowered midway, and one that is not
+    for s in (np.logspace(-6, 6, cin), np.logspace(6, -6, cin)):  # rising and falling
         xs = x * s.astype(np.float32)[:, None, None]
         assert rel_err(_run(engine, kind, xs, wt), _ref(kind, xs, wt)) < TOL
 

@@ -1,12 +1,12 @@
-"""The two-dimensional Winograd F(2x4, 3x3) kernel on split f16 products, where
-it can go wrong: the edges of its 4-row x 64-pixel blocks (planes one row or
+"""The two-dimensional Winograd F(2x4, 3x3) kernel on three bf16 parts, where it
+can go wrong: the edges of its 4-row x 64-pixel blocks (planes one row or
 pixel past them, widths that are and are not multiples of 4, whose columns the
 lanes take from their neighbours), ragged channels against its 8- and
 16-channel groups, and the range of the values.
 
-Tolerance: a split product is within 2^-22 + 2^-22 of the f32 one and the sum
-of up to 100 * 9 of them is rounded in f32 as before, so the 1e-5 relative
-bound of the other operator tests holds with the same margin, at any scale."""
+Tolerance: a product in parts is within 2^-23 of the f32 one and the sum of up
+to 100 * 9 of them is rounded in f32 as before, so the 1e-5 relative bound of
+the other operator tests holds with the same margin, at any scale."""
 import numpy as np
 import pytest
 
@@ -45,7 +45,7 @@ def test_any_magnitude(w42, cin, cout, h, w):
     for sx, sw in ((1.0, 1.0), (2.0**-90, 2.0**20), (2.0**60, 2.0**-30)):
         got = w42.op_conv2d(x * np.float32(sx), wt * np.float32(sw))
         assert rel_err(got.astype(np.float64) / (sx * sw), ref) < TOL
-    for s in (np.logspace(-6, 6, cin), np.logspace(6, -6, cin)):  # a scale lowered midway, and one that is not
+    for s in (np.logspace(-6, 6, cin), np.logspace(6, -6, cin)):  # rising and falling
         xs = x * s.astype(np.float32)[:, None, None]
         assert rel_err(w42.op_conv2d(xs, wt), _ref(xs, wt)) < TOL
 
