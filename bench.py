@@ -7,11 +7,11 @@ blurred-noise image with a ~25% brush-stroke mask.  A "step" is one forward
 pass; the input tensor is resident in HBM before the timed region starts.
 
 Prints one JSON line: passes/s, the roofline of the dominant kernel (the FFC
-3x3 convolutions as Winograd F(4,3) along x, F(2x4, 3x3) on the bottleneck
-planes of 1024x1024 inputs and up: the FLOPs of that algorithm's MFMA
+3x3 convolutions as Winograd F(4,3) along x, F(2x4, 3x3) on large bottleneck
+planes, 2048x2048 inputs among them: the FLOPs of that algorithm's MFMA
 products per launch / mean launch time on the device clock, against the peak
-of FP32 products on the matrix cores that the kernel uses: a third of the
-dense f16 rate, as each is three f16 MFMAs; the direct-convolution equivalent
+of FP32 products on the matrix cores that the kernel uses: a sixth of the
+dense bf16 rate, as each is six bf16 MFMAs; the direct-convolution equivalent
 rate beside it), the host enqueue time of one pass, the wall time of the lama-inpaint
 command on the reference's published case (2048x2048 image, 300x300 hole,
 whole image and --tile) beside the reference's own figures, and the CPU
@@ -33,7 +33,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_FP32_MFMA = 157.3  # TFLOP/s, MI355X dense FP32 matrix
-PEAK_SPLIT = 2500.0 / 3  # FP32 products as three f16 MFMAs each (dense f16: 2.5 PFLOP/s)
+PEAK_SPLIT = 2500.0 / 6  # FP32 products as six bf16 MFMAs each (dense bf16: 2.5 PFLOP/s)
 PEAK_HBM = 8000.0  # GB/s
 # The reference's only published timings of this path (README.md:78-79): one
 # run of its binary on a 2048x2048 image with a 300x300 hole, whole image and
@@ -147,7 +147,7 @@ def main():
     # (family conv3x3g2l), one kernel
     dom_fams = ["conv3x3", "conv3x3g2l"]
     # the FFC 3x3 convolutions run as Winograd F(4,3) along x, or F(2x4, 3x3)
-    # on bottleneck planes of 128 x 128 and up (LAMA_FFC_WINO=2: F(2,3); 0:
+    # on large bottleneck planes (LAMA_FFC_WINO=2: F(2,3); 0:
     # the direct implicit GEMM; 4 / 42 force one Winograd form everywhere).
     # The engine counts each launch's direct-convolution FLOPs, 2 Cin Cout 9 H
     # W; the algorithm's own MFMA products are the fraction `issued` of that:
@@ -164,7 +164,7 @@ def main():
              "lama_conv3x3w4n": "4 rows x 32 px", "lama_conv3x3w4q": "8 rows x 16 px",
              "lama_conv3x3w42": "4 rows x 64 px"}[dom_kernel]
     geometry = "workgroups of 64 channels x " + block
-    # the two default algorithms multiply split f16 halves, the others f32
+    # the two default algorithms multiply in three bf16 parts, the others in f32
     peak = PEAK_SPLIT if wino in (4, 42) else PEAK_FP32_MFMA
     method = {0: "direct implicit GEMM", 2: "Winograd F(2,3) along x", 4: "Winograd F(4,3) along x",
               42: "Winograd F(2x4, 3x3)"}[wino]
