@@ -26,8 +26,10 @@
 #define LAMA_SCRATCH_BYTES (192u << 20)
 // LDS bytes of the two ping-pong buffers of a split-mode FFT block (row pairs
 // or columns per block = this / (2 * 8 * plane side)).  32 KB rather than 64:
-// a block then fits on a CU beside the FFC GEMM's two workgroups (51 KB each),
-// so the side stream's transforms are not held back by that GEMM's launches.
+// two blocks then fit on a CU beside two F(4,3) workgroups (38 KB each), with
+// 64 KB one.  (Beside an F(2x4, 3x3) workgroup, 148 KB, neither fits.)  ms a
+// pass, 32 / 64 KB: 768x768 7.09 / 7.64, 1024x1024 9.49 / 9.58, 1080x1920 19.7 /
+// 20.1; with F(2x4, 3x3) 2048x2048 36.3 / 36.2, 1536x1536 22.2 / 21.9.
 #ifndef LAMA_FFT_SPLIT_LDS
 #define LAMA_FFT_SPLIT_LDS (32 * 1024)
 #endif
@@ -46,9 +48,8 @@
 
 // Complex values per ping-pong buffer of the single-block FFT kernels: the
 // row-pair layout [(h+1)/2][w] or the half spectrum [h][w/2+1], rounded up to
-// even so the second buffer is 16-byte aligned.  (Padding the rows against
-// bank conflicts would cost LDS: at 512x512 a plane's 34 KB must stay within
-// what two FFC GEMM workgroups leave free on a CU -- 37 KB measured slower.)
+// even so the second buffer is 16-byte aligned.  (Rows are not padded against
+// bank conflicts: conflict-free, XOR-swizzled rows measured the same.)
 static inline constexpr int lama_fft_nb(int h, int w)
 {
     const int a = (h + 1) / 2 * w, b = h * (w / 2 + 1);
@@ -280,8 +281,8 @@ struct TailArgs {
 // src0 [M][C0][9], the rest from src1 [M][C - C0][9] (the FFC's local GEMM
 // concatenates l2l and g2l along K).  kind 4: the F(4,3) layout of
 // lama_conv3x3w4*; kind 42: the F(2x4, 3x3) layout of lama_conv3x3w42; kind 1:
-// W[M][C] for lama_conv1x1* (C0 == C).  All hold three bf16 parts of every value (split.h).  dst is pre-zeroed (rows
-// past M, channels past C stay zero).
+// W[M][C] for lama_conv1x1* (C0 == C).  All hold three bf16 parts of every
+// value (split.h).  dst is pre-zeroed (rows past M, channels past C stay zero).
 struct WinoPackJob {
     const float *src0, *src1;
     float *dst;

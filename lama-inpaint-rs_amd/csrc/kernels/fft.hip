@@ -694,7 +694,7 @@ extern "C" __global__ void __launch_bounds__(LAMA_FFT_NT) lama_irfft2_rows(const
 // 75x75) use the single-block algorithm above with every length, count and
 // stride a compile-time constant, so no index arithmetic is left in the
 // kernels but shifts, masks and multiplies-high by constants.  This matters
-// beside the FFC GEMM: its FP32 MFMAs hold the SIMDs' math pipes, and every
+// beside the FFC GEMM: its MFMAs hold the SIMDs' math pipes, and every
 // VALU instruction of these kernels then waits its turn, so the runtime
 // integer divisions of the generic path (about half of its instructions)
 // cost more than the butterflies themselves.  The radix plan is the host's
@@ -837,15 +837,15 @@ __device__ __forceinline__ float2 ct_twiddle_fetch(const FftArgs &A)
 }
 
 // IP: one plane buffer instead of two (passes and reorderings in place
-// through registers), for planes whose two buffers would keep a block from
-// sharing a CU with two FFC GEMM workgroups
+// through registers): half the LDS, 24 KB at 75 x 75.  600x600: 4.41 ms a pass,
+// with two buffers 4.42.
 // ---- 64-point rows as wavefront-shuffle FFTs --------------------------------
 //
 // lama_rfft2_64s / lama_irfft2_64s (the plan takes them with LAMA_FFT64_SHFL=1;
-// the default keeps the LDS passes, which measured faster beside the FFC GEMM:
-// 286.5 against 285.0 passes/s at 512 x 512, while alone these are 7% and 13%
-// faster -- the lane moves are VALU instructions, which wait behind the GEMM's
-// MFMAs, where LDS accesses do not).  A row pair's 64-point transform runs in the
+// the default keeps the LDS passes: a 512x512 pass takes 3.09 ms with either,
+// though alone these are 7% and 13% faster -- the lane moves are VALU
+// instructions, which wait behind the FFC GEMM's MFMAs, where LDS accesses do
+// not).  A row pair's 64-point transform runs in the
 // registers of 16 lanes of one wave, four values per lane, with no LDS pass
 // and no barrier: the index is split as x = 4 l + m (lane l, register m).
 // Forward (natural input): a 16-point DIF transform across the 16 lanes for

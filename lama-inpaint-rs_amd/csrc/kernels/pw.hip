@@ -26,8 +26,10 @@
 // at 192 and 384 channels.
 // lama_conv1x1, lama_conv1x1_res: 64 channels x 64 pixels in fills of 96, the
 // larger planes, where the weights feed twice the pixels and three workgroups a
-// CU cover each other's loads.  256 x 256 plane, alone: conv1 106.7 / 82.3 us
-// (in a 1024 x 1024 pass 47 us; 96-channel tiles of six waves 52).
+// CU cover each other's loads (conv1 in a 1024 x 1024 pass 47 us; 96-channel tiles
+// of six waves 52).  256 x 256 plane, alone, f32 MFMAs / here: conv1 95 / 69 us,
+// the FU conv 95 / 73, conv2 134 / 115.  Nothing is saturated there: MFMAs 0.3
+// busy, an L1 access every third cycle.
 #include <hip/hip_runtime.h>
 
 #include "common.h"

@@ -617,11 +617,10 @@ bool is_pow2(int n) { return n > 0 && (n & (n - 1)) == 0; }
 
 // Plane stride of the bottleneck activations and of the stacked spectrum:
 // the plane length rounded up to a multiple of 4 floats, so that every plane
-// of a 256-byte aligned buffer is 16-byte aligned and the float4 kernels run
-// on planes of any length (75 x 75 = 5625, 75 x 38 = 2850 at 600 x 600).
-// The padding floats are never read as data: the pointwise kernels' last
-// float4 run of a plane feeds only output columns past the plane, which are
-// not stored, and the transforms and 3x3 convolutions index rows.
+// of a 256-byte aligned buffer is 16-byte aligned and finalize works in whole
+// float4 groups on planes of any length (75 x 75 = 5625, 75 x 38 = 2850 at
+// 600 x 600).  Nothing reads the padding floats: the pointwise kernels clamp a
+// pixel to the plane, the transforms and 3x3 convolutions index rows.
 size_t pad4(size_t n) { return (n + 3) & ~(size_t)3; }
 
 }  // namespace
@@ -1090,12 +1089,10 @@ hipFunction_t Engine::conv_fn(int family, const ConvProblem *probs, size_t n, in
 // F(4,3) blocks of 32 Winograd tiles: 2 rows x 64 pixels (lama_conv3x3w4),
 // 4 x 32 (w4n) or 8 x 16 (w4q).  The shape that covers the plane with the
 // fewest blocks, 2 x 64 on a tie; LAMA_W4_TILE=64, 32 or 16 (read at open)
-// forces one.  Measured with the current kernels (passes/s, 64 / 32-pixel
-// blocks, each as many blocks): 512x512 281.2 / 277.8-278.0, 1024x1024
-// 79.7-80.1 / 77.6-77.7, 2048x2048 20.63-20.71 / 20.43-20.54; 600x600 (76 /
-// 57 / 50 blocks of 64 / 32 / 16 pixels) 148.8 / - / 166.4.  (With the
-// LDS-staged weights and 64 x 64 pointwise tiles 2 x 64 had been the
-// slowest: 512x512 228.7 vs 253.6.)
+// forces one.  Measured, ms a pass with blocks of 64 / 32 / 16 pixels: 600x600
+// (76 / 57 / 50 blocks a plane) 5.19 / 4.48 / 4.41, 1080x1920 (272 / 272 / 255)
+// 19.92 / 19.72 / 19.54; as many of each: 512x512 3.09 / 3.08 / 3.10, 1024x1024
+// 9.39 / 9.34 / 9.42.
 int Engine::w4_variant(int OH, int OW) const
 {
     if (w4_force_ == 64) return 0;
@@ -1211,12 +1208,10 @@ int Engine::wino_for(int h8, int w8) const
 
 // Groups of 4 elements per finalize thread (1 or 2): two where one group per
 // thread would give fewer blocks than CUs or between 2.5 and 4 per CU.
-// Measured: at 32 x 32 (128 blocks with one group) two groups gave 448.8-450.4
-// vs 431.3-437.1 passes/s; at 75 x 75
-// 768 blocks ran slower beside the concurrent kernels than 384 (157.4 vs
-// 158.9 passes/s); at 64 x 64 512 blocks ran faster than 256 (260.2 vs
-// 258.5); at 128 x 128 and 256 x 256 planes (8 and 32 blocks per CU) one
-// group was as fast or 0.3% faster.
+// The line was drawn beside the FP32 GEMMs (32 x 32 planes, two groups / one:
+// 449 / 434 passes/s; 75 x 75 158.9 / 157.4; 64 x 64 258.5 / 260.2).  Beside the
+// present ones the two are within 0.4% (ms a pass, one / two: 256x256 1.93 / 1.93,
+// 512x512 3.09 / 3.09, 600x600 4.41 / 4.43, 1024x1024 9.38 / 9.39).
 int Engine::fin_groups(size_t plane) const
 {
     if (fin_groups_force_ == 1 || fin_groups_force_ == 2) return fin_groups_force_;
@@ -1231,9 +1226,10 @@ int Engine::fin_groups(size_t plane) const
 // into s K slices of raw partials that the single-block transform sums (with
 // the BN + ReLU) while loading them.  The largest s of 1, 2, 4 that keeps the
 // launch within LAMA_PW_KSPLIT_WG workgroups, one per CU; 1 with split-mode
-// transforms.  Measured (passes/s, split / unsplit): 256x256 (s = 4) 411.2 /
-// 384.7; 512x512 with s = 2 (two workgroups per CU) 241.8 / 253.1, so 512x512
-// stays unsplit.  LAMA_PW_KSPLIT=1, 2 or 4 (read at open) forces s.
+// transforms.  Measured, ms a pass with s = 1 / 2 / 4: 64x64 1.84 / 1.75 / 1.67
+// and 128x128 1.89 / 1.76 / 1.70 (s = 4 taken), 256x256 2.03 / 1.94 / 1.99 (2),
+// 376x504 3.33 / 3.60 / 3.93 and 512x512 3.08 / 3.30 / 3.54 (1).
+// LAMA_PW_KSPLIT=1, 2 or 4 (read at open) forces s.
 #ifndef LAMA_PW_KSPLIT_WG
 #define LAMA_PW_KSPLIT_WG LAMA_CUS
 #endif
@@ -1585,8 +1581,7 @@ bool Engine::build_plan(Plan &p, void *arena, std::string &err)
                  family != F_CONV1))
                 bad_problem = true;
         }
-        // the head kernels walk their tiles: three (register weights) or two
-        // (weights in LDS) resident workgroups per CU
+        // the head kernels walk their tiles: two resident workgroups per CU
         L.grid = family == F_CONV7 ? std::min(nb, 2u * LAMA_CUS) : nb;
         L.shmem = (family == F_CONV3 || family == F_CONV3G) && wm == 4 ? w4_shmem : 0;
         L.block = block_threads(L.fn);
@@ -2199,11 +2194,13 @@ bool Engine::use_graph(const Plan &p) const
 {
     // LAMA_GRAPH=1 / 0 forces the replayed graph on / off.  By default it is
     // used for inputs of at most 256 x 256, where issuing the pass's launches
-    // one by one takes the host nearly as long as the device takes to run
-    // them (256x256: 1.93-2.13 ms of enqueue against a 2.2 ms pass; one graph
-    // launch enqueues in 0.93 ms), so a slower host would make the pass
-    // host-bound.  Above that the device time dominates and the per-launch
-    // streams measured slightly faster (512x512: 282.2 vs 280.2 passes/s).
+    // one by one takes the host as long as the device takes to run them
+    // (256x256: 1.96-2.07 ms of enqueue, one graph launch 0.97 ms).  Measured,
+    // streams / graph, ms a pass back to back: 128x128 2.02 / 1.70, 256x256
+    // 2.11 / 1.93.  Above that the device time dominates and the two are the
+    // same (256x384 2.38 / 2.39, 384x384 2.62 / 2.62, 512x512 3.09 / 3.08,
+    // 600x600 4.42 / 4.42, 1024x1024 9.47 / 9.46), a lone pass is faster with
+    // streams at the smallest (256x384 2.30 / 2.40), and streams need no capture.
     // Profiled and timeline passes always take the per-launch path.
     if (prof_mask_ != 0 || timeline_ || p.graph_failed) return false;
     if (const char *g = getenv("LAMA_GRAPH")) return atoi(g) == 1;

@@ -302,7 +302,7 @@ private:
     hipFunction_t fn_finalize_g2_[3] = {};  // the same three with two element groups per thread
     hipFunction_t fn_edge_q_[2] = {};       // lama_conv3x3s2_q (8 x 16 tiles), lama_convt_q (4 x 16)
     hipFunction_t fn_head_r_ = nullptr;     // lama_conv7x7r (the 4 -> 64 head, weights in registers)
-    hipFunction_t fn_pw_kh_[2] = {};        // lama_conv1x1_kh, lama_conv1x1_res_kh (64 x 32 K-half tiles)
+    hipFunction_t fn_pw_kh_[2] = {};        // lama_conv1x1_kh, lama_conv1x1_res_kh (96 x 32 K-half tiles)
     bool head_r_ = true;                    // LAMA_HEAD_R=0: the head through lama_conv7x7 (weights in LDS)
     hipFunction_t fn_convt_rows_[2] = {};   // lama_convt_rows (4 x 32 positions), lama_convt_rows_q (8 x 16)
 
