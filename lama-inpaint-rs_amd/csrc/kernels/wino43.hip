@@ -314,8 +314,8 @@ __device__ __forceinline__ void w43_tile(const ConvProblem &P_mem, int b, b8 *vs
 // order (x = i mod 8; the n blocks split as q = n / 8 per XCD, the first
 // r = n mod 8 XCDs one more), so that each XCD works through one contiguous
 // range: with M-block-major problems that is one or two M blocks' weights
-// (0.6 MB each) and one problem's input channels per L2, instead of every
-// M block's weights (A: 4.7 MB against a 4 MB L2) or all 384 global input
+// (0.9 MB each) and one problem's input channels per L2, instead of every
+// M block's weights (A: 7.1 MB against a 4 MB L2) or all 384 global input
 // planes (B: 6.3 MB) in every L2.
 namespace {
 __device__ __forceinline__ int wino_xcd_order(int i, int n)

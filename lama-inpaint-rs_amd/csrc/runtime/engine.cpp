@@ -2201,6 +2201,8 @@ bool Engine::use_graph(const Plan &p) const
     // same (256x384 2.38 / 2.39, 384x384 2.62 / 2.62, 512x512 3.09 / 3.08,
     // 600x600 4.42 / 4.42, 1024x1024 9.47 / 9.46), a lone pass is faster with
     // streams at the smallest (256x384 2.30 / 2.40), and streams need no capture.
+    // (In a process whose other streams leave two of the engine's on one of HIP's
+    // four hardware queues the graph is faster there too: 512x512 3.70 / 3.13.)
     // Profiled and timeline passes always take the per-launch path.
     if (prof_mask_ != 0 || timeline_ || p.graph_failed) return false;
     if (const char *g = getenv("LAMA_GRAPH")) return atoi(g) == 1;
