@@ -45,9 +45,9 @@ def cli_wall_times(H, wpath, tmp, reps=3):
     """Wall time of this build's lama-inpaint on the reference's published case:
     a 2048x2048 image with a seeded 300x300 hole, whole image and --tile, each
     a fresh process (start-up, weight file read, packing and upload, PNG
-    decode and encode included), `reps` runs each.  Beside them, configs[4]'s
-    other case, for which the reference publishes no time: --sections on the
-    same image with a seeded 1024x1024 hole (16 passes of 512x512)."""
+    decode and encode included), `reps` runs each.  Beside them, a case for
+    which the reference publishes no time: --sections on the same image with a
+    seeded 1024x1024 hole (16 passes of 512x512)."""
     cli = os.path.join(ROOT, "lama-inpaint-rs_amd", "bin", "lama-inpaint")
     img = H.synth_image(2048, 2048, 1)
     mask, _ = H.synth_mask_rect(2048, 2048, 300, 300, 2)
@@ -80,7 +80,7 @@ def cli_wall_times(H, wpath, tmp, reps=3):
                      "seeded 300x300 hole (README.md:78-79's case), synthetic weights; wall time of each "
                      f"process, median of {reps}; the reference's figures are its README's, on a GTX 1080; "
                      "sections_1024_hole_s: --sections on the same image with a seeded 1024x1024 hole "
-                     "(BASELINE configs[4], 16 passes of 512x512; no published reference time)")}
+                     "(16 passes of 512x512; no published reference time)")}
 
 
 def main():
@@ -223,7 +223,7 @@ def main():
     host_f32_io = n_io / (time.perf_counter() - t)
     assert np.array_equal(host_out, out)
 
-    # BASELINE configs[2]: the SpectralTransform alone, FFCs 0..17 (distinct
+    # the SpectralTransform alone, FFCs 0..17 (distinct
     # weights) on 384 x (S/8)^2 N(0,1) inputs resident in HBM, back to back
     # on one stream
     h8 = S // 8
@@ -315,7 +315,7 @@ def main():
                 ts.append(time.perf_counter() - t)
             return ts
 
-        # the workload size, median of three; 256x256 (configs[0]'s shape) beside it
+        # the workload size, median of three; 256x256 beside it
         cpu_ts = cpu_passes(cs)
         cpu_s = float(np.median(cpu_ts))
         cpu_ts256 = cpu_passes(256) if cs != 256 else cpu_ts
@@ -363,9 +363,7 @@ def main():
         "vs_baseline": None,
         "dtype": "f32",
         "data": "synthetic (seeded random-init Big-LaMa weights, blurred-noise image, brush-stroke mask)",
-        "config": {"workload": f"Big-LaMa generator whole-image pass {S}x{S}, batch 1"
-                               + {512: " (BASELINE configs[3])", 2048: " (BASELINE configs[4])",
-                                  256: " (BASELINE configs[0] shape)"}.get(S, ""),
+        "config": {"workload": f"Big-LaMa generator whole-image pass {S}x{S}, batch 1",
                    "h": S, "w": S, "mask_coverage": round(coverage, 4), "launches_per_pass": eng.launch_count(S, S)},
         "roofline": {"bound": "mfma",
                      "kernel": (dom_kernel + f" (FFC 3x3 convolutions as {method}, {geometry}"
@@ -405,7 +403,7 @@ def main():
         "host_enqueue_note": ("host time of forward_device (the launch loop alone, device idle at the call), "
                               "median; isolated_pass_ms: the same call through its synchronize"),
         "spectral_block_us": round(spec_us, 2),
-        "spectral_block_workload": f"BASELINE configs[2]: SpectralTransform of FFCs 0..17 on 384x{h8}x{h8}, "
+        "spectral_block_workload": f"SpectralTransform of FFCs 0..17 on 384x{h8}x{h8}, "
                                    "conv1 -> rfft2 -> FU conv -> irfft2 -> conv2, one stream",
         "per_family": per_family,
         "cpu_baseline": cpu,

@@ -25,7 +25,7 @@ def pkg():
 
 @pytest.fixture(scope="session")
 def weights_dir(tmp_path_factory):
-    """Synthetic Big-LaMa containers: `plain` (the BASELINE fixture, seed 0)
+    """Synthetic Big-LaMa containers: `plain` (seed 0)
     and `cal` (the same weights with calibrated BN statistics)."""
     import oracle_api as O
 

@@ -316,7 +316,7 @@ def test_plan_rejects_unsupported_shapes(pkg, engine):
 
 @pytest.mark.gpu
 def test_cli_sections_config4_2048_with_1024_hole(H, engine, tmp_path, weights_dir):
-    """BASELINE configs[4] --sections as specified: a 2048 x 2048 image with a
+    """--sections at its full size: a 2048 x 2048 image with a
     seeded 1024 x 1024 hole, filled as 16 sections of 256 x 256 in 512 x 512
     windows, rim inward; bit-exact with the restated pass loop."""
     img = H.synth_image(2048, 2048, 1)
@@ -335,7 +335,7 @@ def test_cli_sections_config4_2048_with_1024_hole(H, engine, tmp_path, weights_d
 
 @pytest.mark.gpu
 def test_cli_tile_config4_2048_with_300_hole(H, engine, tmp_path, weights_dir):
-    """BASELINE configs[4] --tile as specified: a 2048 x 2048 image with a
+    """--tile at its full size: a 2048 x 2048 image with a
     seeded 300 x 300 hole runs one 600 x 600 window (tile_rect, main.rs:740-777;
     the README's --tile timing is this window).  The output is bit-exact with
     crop-run-paste (main.rs:378-443) restated over the engine; the window's

@@ -1,4 +1,4 @@
-"""the per-layer conv GEMM suite at the 512x512 shapes,
+"""The per-layer conv GEMM suite at the 512x512 shapes,
 FP32, batch 1, N(0,1) activations and He-normal weights, each with its fused
 BN + ReLU epilogue, kernel by kernel against the CPU oracle's direct sums
 (cpu.rs:110-168 for the convolutions, cpu.rs:328-374 for the transposed ones,
@@ -12,12 +12,11 @@ cpu.rs:66-76 and 376-382 for BN and ReLU):
 - the three stride-2 transposed convs 512 -> 256 (64 -> 128), 256 -> 128
   (128 -> 256) and 128 -> 64 (256 -> 512).
 
-Beside them, the FFC 3x3 at the 256-wide planes of a 2048x2048 input
-(configs[4]'s bottleneck), which the forward otherwise runs only inside the
+Beside them, the FFC 3x3 at the 256-wide planes of a 2048x2048 input, which the forward otherwise runs only inside the
 whole pass.
 
 Tolerance: 1e-5 relative L2 (FP32 products, FP32 sums in another order than
-the oracle's sequential loop), 100x inside the north star's 1e-3 per layer.
+the oracle's sequential loop), 100x inside the 1e-3 allowed per layer.
 """
 import numpy as np
 import pytest

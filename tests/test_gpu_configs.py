@@ -1,17 +1,17 @@
-"""BASELINE.json's configurations, each built exactly as specified, on the GPU
+"""The backend's standing workloads, each built exactly as specified, on the GPU
 against the CPU oracle:
 
-* configs[3] (the bench workload): 512x512, the brush-stroke mask that
+* the bench workload: 512x512, the brush-stroke mask that
   bench.py draws (synth_mask_strokes(0.25, seed 2)), blurred-noise image
   seed 1, the seed-0 weights -- both as bench.py loads them (plain BN
   statistics) and with calibrated BN statistics;
-* configs[0]: 256x256 with one seeded 64-wide x 96-tall rectangle, plain and
+* 256x256 with one seeded 64-wide x 96-tall rectangle, plain and
   calibrated weights;
-* configs[2]: the SpectralTransform alone, 18 blocks with distinct weights on
+* the SpectralTransform alone, 18 blocks with distinct weights on
   384 x 64 x 64 N(0,1) inputs, every stage of each block.
 
 Whole passes are checked at every plan step (relative L2 error <= 1e-3, the
-north star's per-layer bound) through lama_hip_forward_steps; the sigmoid
+per-layer bound) through lama_hip_forward_steps; the sigmoid
 output value by value (within 1/255 wherever its pre-activation is
 well-conditioned, see _check_output); and the production path
 (lama_hip_forward: three streams, no step synchronisation) must equal the
@@ -108,7 +108,7 @@ def test_config3_bench_workload_512(pkg, engine, plain_engine, oracles, weights,
     mask, cov = H.synth_mask_strokes(512, 512, 0.25, 2)
     assert 0.2 < cov < 0.3
     eng = plain_engine if kind == "plain" else engine
-    flips = _check_pass(pkg, eng, oracles[kind], weights[kind], img, mask, f"configs[3] {kind}")
+    flips = _check_pass(pkg, eng, oracles[kind], weights[kind], img, mask, f"512x512 {kind}")
     if kind == "cal":
         assert flips == 0
 
@@ -121,20 +121,20 @@ def test_config0_256_rect_64x96(pkg, engine, plain_engine, oracles, weights, kin
     assert mask.sum() // 255 == 64 * 96
     assert mask[y0:y0 + 96, x0:x0 + 64].all()
     eng = plain_engine if kind == "plain" else engine
-    flips = _check_pass(pkg, eng, oracles[kind], weights[kind], img, mask, f"configs[0] {kind}")
+    flips = _check_pass(pkg, eng, oracles[kind], weights[kind], img, mask, f"256x256 {kind}")
     if kind == "cal":
         assert flips == 0
 
 
 def test_config2_spectral_transform_18_blocks(plain_engine, oracles):
-    """configs[2]: FFCs 0..17 (model.5.conv1 .. model.13.conv2), each on its
+    """FFCs 0..17 (model.5.conv1 .. model.13.conv2), each on its
     own seeded N(0,1) 384 x 64 x 64 input: f, spectrum, FU conv, f + ifft
     and the output each within 1e-3 of the oracle."""
     net = oracles["plain"]
     names = ["f", "spectrum", "fu", "f+ifft"]
     for k in range(18):
         x = np.random.default_rng(1000 + k).standard_normal((384, 64, 64)).astype(np.float32)
-        print(f"case configs[2] block {k}", flush=True)
+        print(f"case spectral block {k}", flush=True)
         ref, ref_st = net.spectral(k, x, stages=True)
         got, got_st = plain_engine.spectral(k, x, stages=True)
         for i in range(4):

@@ -1,5 +1,5 @@
 """The whole forward on the GPU against the CPU oracle: every plan step
-within 1e-3 relative L2 error (the north star's per-layer bound), the final
+within 1e-3 relative L2 error (the per-layer bound), the final
 8-bit composite within 1/255 max and 0.1 levels mean, unmasked pixels
 bit-exact."""
 import numpy as np
@@ -125,7 +125,7 @@ def test_g2l_stream_matches_single_order(pkg, engine, monkeypatch, h, w):
 
 
 def test_forward_plain_weights(pkg, weights_dir):
-    """The BASELINE fixture as specified (uncalibrated BN statistics, so the
+    """The plain fixture (uncalibrated BN statistics, so the
     activations grow by ~1e10 through the resblocks): per-step relative error
     still within 1e-3."""
     eng = pkg.hip_engine.Engine()
@@ -229,7 +229,7 @@ def test_forward_512_shuffle_row_fft(pkg, engine, monkeypatch):
 
 
 def test_forward_2048_whole_image(pkg, engine):
-    """configs[4] at its full size (bottleneck 512 x 256 x 256): checked by
+    """2048 x 2048, the largest pass (bottleneck 512 x 256 x 256): checked by
     size-independent properties -- finite, bitwise repeatable, sigmoid range,
     unmasked pixels of the composite bit-exact."""
     h = w = 2048
@@ -250,7 +250,7 @@ def test_forward_2048_whole_image(pkg, engine):
 
 @pytest.mark.timeout(900)
 def test_forward_2048_whole_image_against_the_oracle(pkg, engine, oracle_cal):
-    """configs[4] whole image at its full size against the CPU oracle
+    """A whole 2048 x 2048 image against the CPU oracle
     (main.rs:212-313 through cpu.rs:741-751): a 2048 x 2048 blurred-noise
     image with a seeded 300 x 300 hole; every plan step within the per-layer
     bound, the composite within 1/255 max and 0.1 levels mean, unmasked pixels
@@ -311,11 +311,11 @@ def test_graph_replays_match_eager(pkg, engine, monkeypatch, h, w):
 
 @pytest.mark.parametrize("h,w", [(600, 600), (600, 592)])
 def test_forward_600_tile_window_non_pow2_bottleneck(pkg, engine, oracle_cal, h, w):
-    """configs[4]'s --tile window: 600 x 600 (75 x 75 bottleneck, FFT lengths
+    """The --tile window: 600 x 600 (75 x 75 bottleneck, FFT lengths
     75 and 38 through the reference's opposite-sign rule) against the oracle,
     every step.  600 x 592 gives bottleneck planes of 5550 and spectral planes
-    of 2850 values: even but not multiples of 4, so every 1x1 convolution
-    (conv1, FourierUnit, conv2 with its epilogue) takes the float2 loads."""
+    of 2850 values: not multiples of 4, so the planes' strides are padded and
+    their last tiles ragged in every 1x1 convolution."""
     img, mask = _case(pkg, h, w, "rect")
     x = pkg.host_api.build_input(img, mask)
     print(f"case {h}x{w} rect", flush=True)

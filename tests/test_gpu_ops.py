@@ -3,7 +3,7 @@
 Tolerance: FP32 MFMA products with FP32 accumulation in a different order
 than the oracle's sequential sum -- relative L2 error <= 1e-5 for the GEMM
 families and the f32 FFT (the oracle's FFT runs in f64), far inside the
-1e-3 per-layer bound the north star states.
+1e-3 per-layer bound of whole passes.
 """
 import numpy as np
 import pytest

@@ -236,7 +236,7 @@ def test_net_load_reports_missing_tensor(cal_weights):
 @pytest.mark.parametrize("k,hw", [(0, (32, 32)), (7, (16, 32)), (35, (32, 16))])
 def test_spectral_block_matches_independent_torch_model(weights_dir, k, hw):
     """or_net_spectral (Spectral::forward, cpu.rs:239-265, the isolated
-    SpectralTransform of BASELINE configs[2]) against the torch model's
+    SpectralTransform) against the torch model's
     SpectralTransform on N(0,1) inputs with the plain fixture weights: every
     LAMA_DUMP_SPECTRAL stage (f, spectrum, FU conv, f + ifft) and the output.
     Power-of-two planes, where torch's FFT sign is the reference's."""
